@@ -305,9 +305,8 @@ TSC_API int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, int3
  * sparse_conv_forward (trispconv/pytorch/functional.py:14-51) and the Triton
  * per-slot kernel (triton_kernels.py:16-135).  Output-stationary: each
  * output row accumulates sum_k feat[nbr[k][o]] @ W[k] in fp32 with k
- * ascending (layers with C_in % 4 == 0 and C_out % 16 == 0 that are not
- * 32x32-tile shapes sum 16 bytes of (slot, channel) products per lane quad
- * and matrix-core step instead; the smallest 32x32-tile layers sum the slots
+ * ascending (layers that are not 32x32-tile shapes sum 16 bytes of (slot,
+ * channel) products per lane quad and matrix-core step instead; the smallest 32x32-tile layers sum the slots
  * of each residue mod 4 apart, then the four partial sums in order), adds
  * bias in fp32 and is rounded once to `dtype`.  No atomics; results are
  * bitwise reproducible and independent of `order`.
@@ -364,9 +363,8 @@ TSC_API int tsc_conv_forward_tile(const void* feat, int32_t dtype, int64_t n_in,
                                   int32_t column_tile, void* out, tsc_stream_t stream);
 
 /* Name of the kernel tsc_conv_forward launches for a layer of this shape
- * ("conv_mfma_kernel", "conv_dma_kernel", "conv_split_kernel",
- * "conv_narrow_kernel" or "conv_valu_kernel"; "" for invalid sizes): what a
- * kernel trace lists it under.  No counterpart in the reference; for profilers and benchmarks. */
+ * ("conv_mfma_kernel", "conv_dma_kernel", "conv_split_kernel" or
+ * "conv_narrow_kernel"; "" for invalid sizes): what a kernel trace lists it under.  No counterpart in the reference; for profilers and benchmarks. */
 TSC_API const char* tsc_conv_kernel_name(int32_t dtype, int32_t c_in, int32_t c_out,
                                          int32_t k_vol, int64_t n_out);
 

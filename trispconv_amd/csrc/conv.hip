@@ -15,18 +15,14 @@
 // every output element is a fixed sequence of fp32 operations, so results are
 // bitwise reproducible and independent of the tile order.
 //
-// Three code shapes share that structure:
+// Two code shapes share that structure:
 //   * mfma: f32/f16/bf16 with C_in a multiple of 16, C_out of 32 and K <= 64
 //     — v_mfma_f32_32x32x16_{f16,bf16} or v_mfma_f32_32x32x2_f32, 4 waves x
 //     (64 rows x BN cols) per tile.
-//   * narrow: the other layers with C_in % 4 == 0 and C_out % 16 == 0 (a
-//     LiDAR encoder's 4 -> 16 first layer, 16-wide outputs, K > 64) —
+//   * narrow: every other layer (a LiDAR encoder's 4 -> 16 or 5 -> 16 first
+//     layer, 16-wide outputs, 20 class scores, K > 64) —
 //     v_mfma_f32_16x16x32_{f16,bf16} or v_mfma_f32_16x16x4_f32 over (slot,
 //     channel) pairs, 16 rows per wave.
-//   * valu: everything else (C_in not a multiple of 4 or C_out not of 16) —
-//     one output row per lane and CO columns per thread, weights read with
-//     wave-uniform addresses, slots skipped when no lane of the wave needs
-//     them.
 //
 // The epilogue adds the bias and, when asked, an eval-mode batch norm and a
 // ReLU (a BatchNorm1d and ReLU following the convolution in a
@@ -44,7 +40,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-enum Path { kValu = 0, kMfma = 1, kNarrow = 2 };
+enum Path { kMfma = 1, kNarrow = 2 };
 
 // Input-channel chunk of one stage: 64 bytes of every gathered row per lane
 // half (64 channels of f16/bf16, 32 of f32), or half that when the channels
@@ -57,21 +53,24 @@ int pick_ck(int dtype, int c_in) {
 int pick_bn(int c_out) { return c_out % 128 == 0 ? 128 : (c_out % 64 == 0 ? 64 : 32); }
 int64_t mfma_chunks(int c_in, int ck) { return ceil_div(c_in, ck); }
 
-// MFMA for every dtype when C_in is a multiple of 16 and C_out of 32 (the
-// slot table of K <= 64 slots fits LDS); the narrow MFMA kernel for the other
-// layers whose channels come in 4-channel pieces and 16-column tiles; VALU
-// otherwise.
+// The 32x32 tile for every dtype when C_in is a multiple of 16 and C_out of 32
+// (the slot table of K <= 64 slots fits LDS); the narrow MFMA kernel for every
+// other width.
 Path pick_path(int dtype, int c_in, int c_out, int K) {
   if (c_in % 16 == 0 && c_out % 32 == 0 && K <= 64) return kMfma;
-  if (c_in % 4 == 0 && c_out % 16 == 0) return kNarrow;
-  return kValu;
+  return kNarrow;
 }
+
+// Channels of a slot in the narrow kernel's reduction: C_in rounded up to
+// whole 4-channel pieces (the padding has zero weights), so that a piece never
+// straddles two slots.
+int narrow_cp(int c_in) { return (c_in + 3) / 4 * 4; }
 
 // Steps of the narrow kernel: 16 bytes of reduction values (slot, channel)
 // per lane quad, i.e. 32 values for f16/bf16 and 16 for f32; the last step is
 // padded with zero weights.
 int64_t narrow_steps(int dtype, int K, int c_in) {
-  return ceil_div((int64_t)K * c_in, 4 * (16 / dtype_bytes(dtype)));
+  return ceil_div((int64_t)K * narrow_cp(c_in), 4 * (16 / dtype_bytes(dtype)));
 }
 
 // ----------------------------------------------------------- weight pack --
@@ -139,18 +138,6 @@ __device__ __forceinline__ float src_weight(const void* w, int dt, int layout, i
   return load_any(w, dt, idx);
 }
 
-__global__ void pack_valu_kernel(const void* w, int w_dt, int layout, int K, int c_in, int c_out,
-                                 float* packed) {
-  const int64_t total = (int64_t)K * c_in * c_out;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int co = e % c_out;
-    const int ci = (e / c_out) % c_in;
-    const int k = e / ((int64_t)c_in * c_out);
-    packed[e] = src_weight(w, w_dt, layout, K, c_in, c_out, k, ci, co);
-  }
-}
-
 // MFMA layout: [k][chunk][c_out/32][u][lane][16/sizeof(T)].  Lane l of a
 // 32-column block n supplies column n*32 + l%32, and for lane half h = l/32
 // the channels c*CK + h*CK/2 + u*(16/sizeof(T)) + 0.. of chunk c: the same
@@ -208,16 +195,18 @@ __device__ __forceinline__ void store_out(void* dst, uint4 v, bool nt) {
 // their loads (64 bytes per lane are read at most).
 __device__ __attribute__((aligned(256))) uint4 g_zero_row[16];
 
-// Narrow layout: [step i][c_out/16][lane][LV], LV = 16 / sizeof(T) values.
-// Lane l of 16-column tile n supplies column n*16 + l%16 and the reduction
-// values r = 4*LV*i + LV*(l/16) + 0..LV-1, r = k * C_in + c for slot k and
-// channel c (zero past K * C_in): the values the A operand's lane l gathers
-// for its row.
+// Narrow layout: [step i][ceil(c_out/16)][lane][LV], LV = 16 / sizeof(T)
+// values.  Lane l of 16-column tile n supplies column n*16 + l%16 and the
+// reduction values r = 4*LV*i + LV*(l/16) + 0..LV-1, r = k * cp + c for slot k
+// and channel c, cp = C_in rounded up to a multiple of 4: the values the A
+// operand's lane l gathers for its row.  Zero past the last slot, the last
+// channel and the last column.
 template <typename T>
 __global__ void pack_narrow_kernel(const void* w, int w_dt, int layout, int K, int c_in,
                                    int c_out, int64_t nsteps, T* packed) {
   constexpr int LV = 16 / (int)sizeof(T);
-  const int nt_all = c_out / 16;
+  const int nt_all = (c_out + 15) / 16;
+  const int cp = (c_in + 3) / 4 * 4;
   const int64_t total = nsteps * nt_all * 64 * LV;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
        e += (int64_t)gridDim.x * blockDim.x) {
@@ -226,90 +215,11 @@ __global__ void pack_narrow_kernel(const void* w, int w_dt, int layout, int K, i
     const int nt = (e / (64 * LV)) % nt_all;
     const int64_t i = e / (64 * LV * (int64_t)nt_all);
     const int64_t r = 4 * LV * i + LV * (lane / 16) + v;
-    const int k = static_cast<int>(r / c_in);
-    const int ci = static_cast<int>(r % c_in);
+    const int k = static_cast<int>(r / cp);
+    const int ci = static_cast<int>(r % cp);
     const int co = nt * 16 + lane % 16;
-    packed[e] = from_f32<T>(k < K ? src_weight(w, w_dt, layout, K, c_in, c_out, k, ci, co) : 0.f);
-  }
-}
-
-// ---------------------------------------------------------------- VALU --
-// VB: bytes of one feature load (16 or 8 when every row is a whole number of
-// such vectors and the features are aligned to them, else one element).
-template <int VB> struct VecOf;
-template <> struct VecOf<16> { using type = uint4; };
-template <> struct VecOf<8> { using type = uint2; };
-template <> struct VecOf<4> { using type = uint32_t; };
-template <> struct VecOf<2> { using type = uint16_t; };
-
-template <typename T, int CO, int VB>
-__global__ void __launch_bounds__(256) conv_valu_kernel(
-    const T* __restrict__ feat, int c_in, const float* __restrict__ W, Epilogue ep,
-    const int32_t* __restrict__ nbr, const int32_t* __restrict__ order, int nbr_ordered,
-    int64_t n_out, int K, int c_out, T* __restrict__ out) {
-  using Vec = typename VecOf<VB>::type;
-  constexpr int NV = VB / (int)sizeof(T);  // values per load
-  static_assert(NV >= 1 && NV * (int)sizeof(T) == VB, "vector of whole elements");
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int co0 = blockIdx.y * CO;
-  const bool valid = t < n_out;
-  __shared__ float s_scale[CO], s_shift[CO];  // the batch norm of this block's columns
-  if (threadIdx.x < CO)
-    channel_affine(ep, co0 + threadIdx.x, s_scale[threadIdx.x], s_shift[threadIdx.x]);
-  __syncthreads();
-  const int64_t o = valid ? (order ? order[t] : t) : 0;
-  float acc[CO];
-#pragma unroll
-  for (int c = 0; c < CO; ++c) acc[c] = 0.f;
-  // Slots go in groups of G: the group's map entries are loaded together, then
-  // for each NV-channel piece the G gathers are issued before any is used, so
-  // a row waits on about K/G load round trips instead of K.
-  constexpr int G = 9;
-  const int64_t col = nbr_ordered ? t : o;  // the map's column of this row
-  for (int k0 = 0; k0 < K; k0 += G) {
-    int32_t j[G];
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      const int k = k0 + u;
-      j[u] = valid && k < K ? (nbr ? nbr[(int64_t)k * n_out + col] : static_cast<int32_t>(o)) : -1;
-    }
-    uint32_t live = 0;  // slots of the group that some lane of the wave uses
-#pragma unroll
-    for (int u = 0; u < G; ++u) live |= (__ballot(j[u] >= 0) != 0ull ? 1u : 0u) << u;
-    if (live == 0) continue;
-    for (int ci0 = 0; ci0 < c_in; ci0 += NV) {
-      Vec v[G];
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        // one vector load through a selected pointer (a conditional load of
-        // the vector gets split into per-element loads)
-        const Vec* src = j[u] >= 0
-                             ? reinterpret_cast<const Vec*>(feat + (int64_t)j[u] * c_in) + ci0 / NV
-                             : reinterpret_cast<const Vec*>(g_zero_row);
-        v[u] = *src;
-      }
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        if (!((live >> u) & 1u)) continue;
-        const float* wk = W + ((int64_t)(k0 + u) * c_in + ci0) * c_out + co0;
-        const T* vals = reinterpret_cast<const T*>(&v[u]);
-#pragma unroll
-        for (int q = 0; q < NV; ++q) {
-          const float xv = to_f32<T>(vals[q]);
-          const float* wr = wk + (int64_t)q * c_out;
-#pragma unroll
-          for (int c = 0; c < CO; ++c) acc[c] = fmaf(xv, wr[c], acc[c]);
-        }
-      }
-    }
-  }
-  if (!valid) return;
-  T* dst = out + o * c_out + co0;
-#pragma unroll
-  for (int c = 0; c < CO; ++c) {
-    const float b = ep.bias ? load_param(ep.bias, ep.bias_dt, co0 + c) : 0.f;
-    dst[c] = from_f32<T>(finish(acc[c] + b, s_scale[c], s_shift[c], ep.mean != nullptr,
-                                ep.relu != 0));
+    const bool in = k < K && ci < c_in && co < c_out;
+    packed[e] = from_f32<T>(in ? src_weight(w, w_dt, layout, K, c_in, c_out, k, ci, co) : 0.f);
   }
 }
 
@@ -1373,15 +1283,27 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
 }
 
 // --------------------------------------------------------- narrow MFMA --
-// Layers with C_in % 4 == 0 and C_out % 16 == 0 that the 32x32 tile does not
-// take.  The reduction runs over r = k * C_in + c (slot k, channel c) in steps
-// of 4*LV values, LV = 16 / sizeof(T): one v_mfma_f32_16x16x32 for f16/bf16,
-// four v_mfma_f32_16x16x4_f32 for f32.  A wave owns 16 output rows and NT
-// 16-column tiles.  Lane l supplies row l%16's values r = 4*LV*i + LV*(l/16)
-// .. +LV-1 of step i, gathered straight from the input rows the map names: one
-// 16-byte piece, or for f16/bf16 with C_in % 8 == 4 two 8-byte pieces of four
-// channels each (the zero row for absent neighbours and the padding past
-// K * C_in).
+// Layers that the 32x32 tile does not take.  The reduction runs over
+// r = k * cp + c (slot k, channel c, cp = C_in rounded up to a multiple of 4)
+// in steps of 4*LV values, LV = 16 / sizeof(T): one v_mfma_f32_16x16x32 for
+// f16/bf16, four v_mfma_f32_16x16x4_f32 for f32.  A wave owns 16 output rows
+// and NT 16-column tiles.  Lane l supplies row l%16's values
+// r = 4*LV*i + LV*(l/16) .. +LV-1 of step i, gathered straight from the input
+// rows the map names (zeros for absent neighbours and padding), in one of
+// three forms:
+//   * kWhole, C_in % 4 == 0 and aligned features: one 16-byte piece, or for
+//     f16/bf16 with C_in % 8 == 4 two 8-byte pieces of four channels each;
+//   * kRagged, any C_in and element-aligned features: the same pieces, read
+//     unaligned.  A piece may run past its row's end (the channels past C_in
+//     are cleared, whatever they hold) but never past the buffer's: it then
+//     starts earlier and is shifted back into place;
+//   * kSingle, feature buffers smaller than one piece: element by element.
+// C_out that is no multiple of 16 has zero-weight columns that are not stored.
+// These widths ran one row per lane on the vector ALU before, 20 class scores
+// with every feature row read by five column groups.  Per pass, before and
+// after: 96 -> 20 f16 over 120k rows 70 -> 21 us; a 3 -> 32 f16 layer with 125
+// slots over 80k rows, with its pair build, 209 -> 130 us; 5 -> 16 and 16 -> 16
+// f16 over 60k LiDAR rows, with the build, 90 -> 81 us.
 // A group of steps loads all its map entries, then all its gathers and
 // weight operands, then runs its MFMAs, so a 3x3x3 layer with C_in = 4 (four
 // steps) costs two dependent memory round trips.  Each output is the same
@@ -1417,9 +1339,52 @@ template <> struct Mfma16<float> {
 
 constexpr int kNarrowRows = 16;  // output rows per wave (the MFMA's M)
 
-__device__ __forceinline__ uint4 join_pieces(const uint4& a, const uint4&) { return a; }
-__device__ __forceinline__ uint4 join_pieces(const uint2& a, const uint2& b) {
-  return make_uint4(a.x, a.y, b.x, b.y);
+enum NarrowRead { kWhole = 0, kRagged = 1, kSingle = 2 };
+
+template <int BYTES> struct VecOf;
+template <> struct VecOf<16> { using type = uint4; };
+template <> struct VecOf<8> { using type = uint2; };
+template <> struct VecOf<4> { using type = uint32_t; };
+template <> struct VecOf<2> { using type = uint16_t; };
+
+// The NP pieces of a lane and step as one operand vector.
+__device__ __forceinline__ uint4 join_pieces(const uint4* v) { return v[0]; }
+__device__ __forceinline__ uint4 join_pieces(const uint2* v) {
+  return make_uint4(v[0].x, v[0].y, v[1].x, v[1].y);
+}
+__device__ __forceinline__ uint4 join_pieces(const uint32_t* v) {
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ uint4 join_pieces(const uint16_t* v) {
+  return make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16,
+                    v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
+}
+
+// Four channels read at the byte address p, of which the first `bytes - shift`
+// bytes after `shift` are wanted: shifted into place, the rest cleared.
+__device__ __forceinline__ uint2 ragged_piece(const char* p, uint32_t shift, uint32_t bytes,
+                                              uint2) {
+  uint64_t v;
+  __builtin_memcpy(&v, p, 8);
+  v >>= 8 * shift;
+  v &= bytes >= 8 ? ~0ull : (1ull << (8 * bytes)) - 1;
+  return make_uint2(static_cast<uint32_t>(v), static_cast<uint32_t>(v >> 32));
+}
+__device__ __forceinline__ uint4 ragged_piece(const char* p, uint32_t shift, uint32_t bytes,
+                                              uint4) {
+  uint4 v;
+  __builtin_memcpy(&v, p, 16);
+  if (shift & 8) v = make_uint4(v.z, v.w, 0u, 0u);
+  if (shift & 4) v = make_uint4(v.y, v.z, v.w, 0u);
+  return make_uint4(bytes > 0 ? v.x : 0u, bytes > 4 ? v.y : 0u, bytes > 8 ? v.z : 0u,
+                    bytes > 12 ? v.w : 0u);
+}
+
+// Sixteen bytes of packed weights, of which only the words need be aligned.
+__device__ __forceinline__ uint4 load_words(const uint4* p) {
+  uint4 v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(reinterpret_cast<const uint32_t*>(p), 4), 16);
+  return v;
 }
 
 // Entry i of a per-channel parameter, or dflt where the pointer is null.  The
@@ -1430,14 +1395,15 @@ __device__ __forceinline__ float param_or(const void* p, int dt, int64_t i, floa
   return p ? v : dflt;
 }
 
-// PIECE: bytes per gather (16 or 8); NT: 16-column tiles per wave.  A group
-// is SG steps: 8 / NT gathers and 32 / NP weight registers per lane.
+// PIECE: bytes per gather (16 or 8, or one element); NT: 16-column tiles per
+// wave.  A group is SG steps: 8 / NT gathers and 32 / NP weight registers per
+// lane.
 // B32: layers whose features and map stay below 2^31 bytes (NarrowB32::fits).
 // The gathers and map loads then go through buffer loads with 32-bit
 // offsets: an offset past the buffer's end reads zeros, which gives absent
 // neighbours their zero row and the identity map (a buffer of no bytes) its
 // zero entries, and the slot of a reduction index is one multiply-high by
-// C_in's rounded-up reciprocal.  The 64-bit addresses and the division cost
+// cp's rounded-up reciprocal.  The 64-bit addresses and the division cost
 // each step about three times the vector instructions (a wave of the 20k-row
 // 16->16 fp32 layer executed 1,623 of them for 108 MFMAs).  Both forms sum
 // the same products in the same order.
@@ -1445,20 +1411,20 @@ struct NarrowB32 {
   uint32_t feat_bytes;  // n_in * C_in * sizeof(T)
   uint32_t map_bytes;   // K * n_out * 4, 0 for the identity map
   uint32_t row_bytes;   // C_in * sizeof(T)
-  uint32_t cin_mag;     // ceil(2^32 / C_in)
+  uint32_t cp_mag;      // ceil(2^32 / cp)
   static bool fits(int64_t n_in, int c_in, int elem, int64_t n_out, int K, int64_t nsteps,
                    int lv) {
     const int64_t r_end = 4 * lv * nsteps;  // reduction indices stay below this
     return n_in * c_in * elem < (int64_t(1) << 31) && (int64_t)K * n_out * 4 < (int64_t(1) << 31) &&
            n_in < (int64_t(1) << 24) && (int64_t)c_in * elem < (int64_t(1) << 24) &&
-           r_end * c_in < (int64_t(1) << 32);
+           r_end * narrow_cp(c_in) < (int64_t(1) << 32);
   }
 };
 constexpr int kBufferWord3 = 0x00020000;  // raw buffer, 32-bit data (gfx9 family)
 
-template <typename T, int PIECE, int NT, bool B32>
+template <typename T, int READ, int PIECE, int NT, bool B32>
 __global__ void __launch_bounds__(256) conv_narrow_kernel(
-    const T* __restrict__ feat, int c_in, const T* __restrict__ W, Epilogue ep,
+    const T* __restrict__ feat, int64_t feat_bytes, int c_in, const T* __restrict__ W, Epilogue ep,
     const int32_t* __restrict__ nbr, const int32_t* __restrict__ order, int nbr_ordered,
     int64_t n_out, int K, int c_out, int nsteps, NarrowB32 nb32, T* __restrict__ out) {
   using Op = Mfma16<T>;
@@ -1467,7 +1433,9 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
   constexpr int VPP = PIECE / (int)sizeof(T);  // values per piece
   constexpr int NP = 16 / PIECE;               // pieces per lane and step
   constexpr int SG = 8 / (NP * NT) > 0 ? 8 / (NP * NT) : 1;
-  static_assert(PIECE == 16 || (PIECE == 8 && sizeof(T) == 2), "8- or 16-byte pieces");
+  static_assert(READ == kSingle ? PIECE == (int)sizeof(T)
+                                : PIECE == 16 || (PIECE == 8 && sizeof(T) == 2), "piece size");
+  static_assert(READ != kRagged || VPP == 4, "a ragged piece is four channels");
   const int lane = threadIdx.x & 63;
   const uint32_t q = lane >> 4;  // which 8 values of a step this lane supplies
   const int rl = lane & 15;      // A row, B and D column of this lane
@@ -1478,8 +1446,9 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
   // its column of the map; lanes past the last row read column 0 (their
   // loads are issued too, and then discarded)
   const int64_t col = va ? (nbr_ordered ? pa : oa) : 0;
-  const int nt_all = c_out / 16;
+  const int nt_all = (c_out + 15) / 16;
   const int nt0 = blockIdx.y * NT;
+  const uint32_t cp = READ == kWhole ? c_in : (c_in + 3) / 4 * 4;
   uint64_t zero_addr = reinterpret_cast<uint64_t>(g_zero_row);
   asm volatile("" : "+s"(zero_addr));
   // global (not flat) loads for both the gathered rows and the zero row
@@ -1492,7 +1461,8 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
   float bias[NT], mean[NT], var[NT], gamma[NT], beta[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
-    const int co = (nt0 + n) * 16 + rl;
+    const int col_n = (nt0 + n) * 16 + rl;
+    const int co = col_n < c_out ? col_n : c_out - 1;  // padding columns are not stored
     bias[n] = param_or(ep.bias, ep.bias_dt, co, 0.f);
     mean[n] = param_or(ep.mean, ep.bn_dt, co, 0.f);
     var[n] = param_or(ep.var, ep.bn_dt, co, 1.f);
@@ -1524,9 +1494,10 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
     for (int u = 0; u < SG * NP; ++u) {
       const int i = i0 + u / NP;
       const uint32_t r = 4u * LV * static_cast<uint32_t>(i) + LV * q + VPP * static_cast<uint32_t>(u % NP);
-      const uint32_t k = B32 ? __umulhi(r, nb32.cin_mag) : r / static_cast<uint32_t>(c_in);
-      ch[u] = r - k * static_cast<uint32_t>(c_in);
-      const bool live = va && i < nsteps && k < static_cast<uint32_t>(K);
+      const uint32_t k = B32 ? __umulhi(r, nb32.cp_mag) : r / cp;
+      ch[u] = r - k * cp;
+      const bool live = va && i < nsteps && k < static_cast<uint32_t>(K) &&
+                        (READ != kSingle || ch[u] < static_cast<uint32_t>(c_in));
       // every lane loads (dead ones from slot K-1 of their column), so the
       // group's map loads issue back to back; dead lanes then use -1
       int32_t e;
@@ -1544,7 +1515,28 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
     Piece v[SG * NP];
 #pragma unroll
     for (int u = 0; u < SG * NP; ++u) {
-      if constexpr (B32) {
+      if constexpr (READ == kSingle) {
+        const T* src = j[u] >= 0 ? feat + (int64_t)j[u] * c_in + ch[u]
+                                 : reinterpret_cast<const T*>(zero_piece);
+        v[u] = __builtin_bit_cast(Piece, *src);
+      } else if constexpr (READ == kRagged) {
+        // the wanted channels of this piece, none of an absent row's; a piece
+        // that would end past the buffer starts earlier (feat_bytes >= PIECE)
+        const uint32_t bytes = j[u] >= 0 ? (static_cast<uint32_t>(c_in) - ch[u]) * (uint32_t)sizeof(T) : 0u;
+        const uint32_t row = j[u] >= 0 ? static_cast<uint32_t>(j[u]) : 0u;
+        if constexpr (B32) {
+          const uint32_t off = __umul24(row, nb32.row_bytes) + ch[u] * static_cast<uint32_t>(sizeof(T));
+          const uint32_t last = nb32.feat_bytes - PIECE;
+          const uint32_t at = off < last ? off : last;
+          v[u] = ragged_piece(reinterpret_cast<const char*>(feat) + at, off - at, bytes, Piece{});
+        } else {
+          const int64_t off = ((int64_t)row * c_in + ch[u]) * (int64_t)sizeof(T);
+          const int64_t last = feat_bytes - PIECE;
+          const int64_t at = off < last ? off : last;
+          v[u] = ragged_piece(reinterpret_cast<const char*>(feat) + at,
+                              static_cast<uint32_t>(off - at), bytes, Piece{});
+        }
+      } else if constexpr (B32) {
         // absent rows read past the buffer's end: zeros
         const uint32_t off = j[u] >= 0 ? __umul24(static_cast<uint32_t>(j[u]), nb32.row_bytes) +
                                              ch[u] * static_cast<uint32_t>(sizeof(T))
@@ -1565,12 +1557,13 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
     for (int u = 0; u < SG; ++u)
 #pragma unroll
       for (int n = 0; n < NT; ++n)
-        b[u][n] = i0 + u < nsteps ? Wv[((int64_t)(i0 + u) * nt_all + nt0 + n) * 64 + lane]
-                                  : make_uint4(0u, 0u, 0u, 0u);
+        b[u][n] = i0 + u < nsteps
+                      ? load_words(Wv + ((int64_t)(i0 + u) * nt_all + nt0 + n) * 64 + lane)
+                      : make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
     for (int u = 0; u < SG; ++u) {
       if (i0 + u >= nsteps) break;
-      const uint4 a = join_pieces(v[u * NP], v[u * NP + NP - 1]);
+      const uint4 a = join_pieces(v + u * NP);
 #pragma unroll
       for (int n = 0; n < NT; ++n) acc[n] = Op::step(a, b[u][n], acc[n]);
     }
@@ -1593,7 +1586,7 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
     const float sh = beta[n] - mean[n] * sc;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (orow[e] >= 0)
+      if (orow[e] >= 0 && co < c_out)
         out[(int64_t)orow[e] * c_out + co] = from_f32<T>(
             finish(acc[n][e] + bias[n], sc, sh, ep.mean != nullptr, ep.relu != 0));
   }
@@ -1739,7 +1732,7 @@ int dispatch_mfma(const void* feat, int c_in, const void* W, const Epilogue& ep,
   return set_error(TSC_EUNSUPPORTED, "conv: no MFMA tile for c_in=%d c_out=%d", c_in, c_out);
 }
 
-template <typename T, int PIECE, int NT>
+template <typename T, int READ, int PIECE, int NT>
 int launch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, const Epilogue& ep,
                   const int32_t* nbr, const int32_t* order, int nbr_ordered, int64_t n_out, int K,
                   int c_out, void* out, hipStream_t s) {
@@ -1747,21 +1740,24 @@ int launch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, const
                      : std::is_same<T, __half>::value ? TSC_F16 : TSC_BF16;
   const int64_t nsteps = narrow_steps(dt, K, c_in);
   TSC_REQUIRE(nsteps < (int64_t(1) << 26), "conv: K * C_in too large");
-  dim3 grid(static_cast<unsigned>(ceil_div(n_out, 4 * kNarrowRows)),
-            static_cast<unsigned>(c_out / 16 / NT));
   constexpr int elem = static_cast<int>(sizeof(T));
+  const int64_t feat_bytes = n_in * c_in * elem;
+  const int64_t cols = ceil_div(c_out, 16) / NT;
+  TSC_REQUIRE(cols < 65536, "conv: C_out too large");
+  dim3 grid(static_cast<unsigned>(ceil_div(n_out, 4 * kNarrowRows)), static_cast<unsigned>(cols));
   if (NarrowB32::fits(n_in, c_in, elem, n_out, K, nsteps, 16 / elem)) {
-    const NarrowB32 nb32{static_cast<uint32_t>(n_in * c_in * elem),
+    const int cp = narrow_cp(c_in);
+    const NarrowB32 nb32{static_cast<uint32_t>(feat_bytes),
                          nbr ? static_cast<uint32_t>((int64_t)K * n_out * 4) : 0u,
                          static_cast<uint32_t>(c_in * elem),
-                         static_cast<uint32_t>(((uint64_t(1) << 32) + c_in - 1) / c_in)};
-    conv_narrow_kernel<T, PIECE, NT, true><<<grid, 256, 0, s>>>(
-        static_cast<const T*>(feat), c_in, static_cast<const T*>(W), ep, nbr, order, nbr_ordered,
-        n_out, K, c_out, static_cast<int>(nsteps), nb32, static_cast<T*>(out));
+                         static_cast<uint32_t>(((uint64_t(1) << 32) + cp - 1) / cp)};
+    conv_narrow_kernel<T, READ, PIECE, NT, true><<<grid, 256, 0, s>>>(
+        static_cast<const T*>(feat), feat_bytes, c_in, static_cast<const T*>(W), ep, nbr, order,
+        nbr_ordered, n_out, K, c_out, static_cast<int>(nsteps), nb32, static_cast<T*>(out));
   } else {
-    conv_narrow_kernel<T, PIECE, NT, false><<<grid, 256, 0, s>>>(
-        static_cast<const T*>(feat), c_in, static_cast<const T*>(W), ep, nbr, order, nbr_ordered,
-        n_out, K, c_out, static_cast<int>(nsteps), NarrowB32{}, static_cast<T*>(out));
+    conv_narrow_kernel<T, READ, PIECE, NT, false><<<grid, 256, 0, s>>>(
+        static_cast<const T*>(feat), feat_bytes, c_in, static_cast<const T*>(W), ep, nbr, order,
+        nbr_ordered, n_out, K, c_out, static_cast<int>(nsteps), NarrowB32{}, static_cast<T*>(out));
   }
   TSC_LAUNCH_CHECK("conv_narrow");
   return 0;
@@ -1771,77 +1767,39 @@ template <typename T>
 int dispatch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, const Epilogue& ep,
                     const int32_t* nbr, const int32_t* order, int nbr_ordered, int64_t n_out,
                     int K, int c_out, void* out, hipStream_t s) {
+  constexpr int elem = static_cast<int>(sizeof(T));
   // Column tiles per wave: up to 4, fewer while that leaves under 2048
   // workgroups (each extra column group re-gathers its rows, from cache).
-  const int nt_all = c_out / 16;
+  const int nt_all = static_cast<int>(ceil_div(c_out, 16));
   const int64_t blocks = ceil_div(n_out, 4 * kNarrowRows);
   int nt = nt_all % 4 == 0 ? 4 : (nt_all % 2 == 0 ? 2 : 1);
   while (nt > 1 && blocks * (nt_all / nt) < 2048) nt /= 2;
-  const int piece = (c_in % 8 == 0 || std::is_same<T, float>::value) ? 16 : 8;
-  TSC_REQUIRE((reinterpret_cast<uintptr_t>(feat) & (piece - 1)) == 0 &&
-                  (reinterpret_cast<uintptr_t>(W) & 15) == 0,
-              "conv: features must be %d-byte and weights 16-byte aligned", piece);
-#define TSC_NARROW_CASE(P_, NT_)                                                             \
-  if (piece == P_ && nt == NT_)                                                              \
-    return launch_narrow<T, P_, NT_>(feat, n_in, c_in, W, ep, nbr, order, nbr_ordered, n_out, K, \
-                                     c_out, out, s);
-  TSC_NARROW_CASE(16, 1)
-  TSC_NARROW_CASE(16, 2)
-  TSC_NARROW_CASE(16, 4)
+  const int whole = (c_in % 8 == 0 || elem == 4) ? 16 : 8;  // bytes of an aligned piece
+  const uintptr_t f = reinterpret_cast<uintptr_t>(feat);
+  TSC_REQUIRE(f % elem == 0, "conv: features must be aligned to their elements");
+  // Widths of whole pieces and tiles are refused features or weights that are
+  // not aligned to them; the others take any that are aligned to elements
+  // (weights: to words), as they always have.
+  const bool regular = c_in % 4 == 0 && c_out % 16 == 0;
+  TSC_REQUIRE(!regular || ((f & (whole - 1)) == 0 && (reinterpret_cast<uintptr_t>(W) & 15) == 0),
+              "conv: features must be %d-byte and weights 16-byte aligned", whole);
+  TSC_REQUIRE((reinterpret_cast<uintptr_t>(W) & 3) == 0, "conv: weights must be 4-byte aligned");
+  constexpr int ragged = 4 * elem;  // bytes of a ragged piece
+  int read = c_in % 4 == 0 && (f & (whole - 1)) == 0 ? kWhole : kRagged;
+  if (read == kRagged && n_in * c_in * elem < ragged) read = kSingle;
+  const int piece = read == kWhole ? whole : read == kRagged ? ragged : elem;
+  if (read == kSingle) nt = 1;
+#define TSC_NARROW_CASE(R_, P_, NT_)                                                            if (read == R_ && piece == P_ && nt == NT_)                                                     return launch_narrow<T, R_, P_, NT_>(feat, n_in, c_in, W, ep, nbr, order, nbr_ordered,                                             n_out, K, c_out, out, s);
+#define TSC_NARROW_CASES(R_, P_)   TSC_NARROW_CASE(R_, P_, 1) TSC_NARROW_CASE(R_, P_, 2) TSC_NARROW_CASE(R_, P_, 4)
+  TSC_NARROW_CASES(kWhole, 16)
   if constexpr (sizeof(T) == 2) {
-    TSC_NARROW_CASE(8, 1)
-    TSC_NARROW_CASE(8, 2)
-    TSC_NARROW_CASE(8, 4)
+    TSC_NARROW_CASES(kWhole, 8)
   }
+  TSC_NARROW_CASES(kRagged, ragged)
+  TSC_NARROW_CASE(kSingle, elem, 1)
+#undef TSC_NARROW_CASES
 #undef TSC_NARROW_CASE
   return set_error(TSC_EUNSUPPORTED, "conv: no narrow tile for c_in=%d c_out=%d", c_in, c_out);
-}
-
-template <typename T, int CO>
-int launch_valu(const void* feat, int c_in, const void* W, const Epilogue& ep,
-                const int32_t* nbr, const int32_t* order, int nbr_ordered, int64_t n_out, int K,
-                int c_out, void* out, hipStream_t s) {
-  dim3 grid(static_cast<unsigned>(ceil_div(n_out, 256)), static_cast<unsigned>(c_out / CO));
-  const int row_bytes = c_in * (int)sizeof(T);
-  const uintptr_t a = reinterpret_cast<uintptr_t>(feat);
-#define TSC_VALU_LAUNCH(VB_)                                                                  \
-  conv_valu_kernel<T, CO, VB_><<<grid, 256, 0, s>>>(static_cast<const T*>(feat), c_in,       \
-                                                    static_cast<const float*>(W), ep, nbr,    \
-                                                    order, nbr_ordered, n_out, K, c_out,      \
-                                                    static_cast<T*>(out))
-  if (row_bytes % 16 == 0 && a % 16 == 0)
-    TSC_VALU_LAUNCH(16);
-  else if (row_bytes % 8 == 0 && a % 8 == 0)
-    TSC_VALU_LAUNCH(8);
-  else
-    TSC_VALU_LAUNCH(sizeof(T));
-#undef TSC_VALU_LAUNCH
-  TSC_LAUNCH_CHECK("conv_valu");
-  return 0;
-}
-
-template <typename T>
-int dispatch_valu(const void* feat, int c_in, const void* W, const Epilogue& ep,
-                  const int32_t* nbr, const int32_t* order, int nbr_ordered, int64_t n_out, int K,
-                  int c_out, void* out, hipStream_t s) {
-  // Columns per thread: the widest that divides c_out, narrowed for small
-  // layers until there are at least 64k threads (a small layer's time is one
-  // thread's chain of slots; narrower threads shorten it, and the repeated
-  // row loads of the column groups hit in cache).
-  int co_max = 32;
-  while (co_max > 4 && n_out * (c_out / co_max) < 65536) co_max /= 2;
-#define TSC_VALU_CASE(CO_)                                                                   \
-  if (CO_ <= co_max && c_out % CO_ == 0)                                                     \
-    return launch_valu<T, CO_>(feat, c_in, W, ep, nbr, order, nbr_ordered, n_out, K,        \
-                               c_out, out, s);
-  TSC_VALU_CASE(32)
-  TSC_VALU_CASE(16)
-  TSC_VALU_CASE(8)
-  TSC_VALU_CASE(4)
-  TSC_VALU_CASE(2)
-  TSC_VALU_CASE(1)
-#undef TSC_VALU_CASE
-  return set_error(TSC_EUNSUPPORTED, "conv: unsupported c_out=%d", c_out);
 }
 
 }  // namespace
@@ -1855,9 +1813,11 @@ extern "C" int64_t tsc_packed_weight_bytes(int32_t k_vol, int32_t c_in, int32_t 
     const int ck = pick_ck(dtype, c_in);
     return (int64_t)k_vol * mfma_chunks(c_in, ck) * ck * c_out * dtype_bytes(dtype);
   }
-  if (pick_path(dtype, c_in, c_out, k_vol) == kNarrow)
-    return narrow_steps(dtype, k_vol, c_in) * (c_out / 16) * 64 * 16;
-  return (int64_t)k_vol * c_in * c_out * 4;
+  const int64_t bytes = narrow_steps(dtype, k_vol, c_in) * ceil_div(c_out, 16) * 64 * 16;
+  // widths that do not fill their pieces and tiles: no less than an fp32
+  // (K, C_in, C_out) copy, the size these weights have always had
+  const int64_t fp32 = (int64_t)k_vol * c_in * c_out * 4;
+  return (c_in % 4 || c_out % 16) && fp32 > bytes ? fp32 : bytes;
 }
 
 extern "C" int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, int32_t k_vol,
@@ -1868,7 +1828,7 @@ extern "C" int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, i
   TSC_REQUIRE(layout == 0 || layout == 1, "pack: layout must be 0 (KRSC) or 1 (flat)");
   TSC_REQUIRE(k_vol > 0 && c_in > 0 && c_out > 0, "pack: sizes must be positive");
   TSC_REQUIRE(w && packed, "pack: null pointer");
-  const int64_t total = (int64_t)k_vol * (c_in + 32) * c_out;  // covers a padded chunk or step
+  const int64_t total = (int64_t)k_vol * (c_in + 32) * (c_out + 15);  // covers padded chunks and tiles
   const int grid = static_cast<int>(ceil_div(total, 256) < 2048 ? ceil_div(total, 256) : 2048);
   const Path path = pick_path(dtype, c_in, c_out, k_vol);
   if (path == kNarrow) {
@@ -1893,9 +1853,6 @@ extern "C" int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, i
     else
       pack_mfma_kernel<__hip_bfloat16><<<grid, 256, 0, s>>>(
           w, w_dtype, layout, k_vol, c_in, c_out, ck, static_cast<__hip_bfloat16*>(packed));
-  } else {
-    pack_valu_kernel<<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out,
-                                          static_cast<float*>(packed));
   }
   TSC_LAUNCH_CHECK("pack_weight");
   return 0;
@@ -1948,24 +1905,14 @@ static int conv_forward(const void* feat, int32_t dtype, int64_t n_in, int32_t c
     return dispatch_mfma<__hip_bfloat16>(feat, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out,
                                          k_vol, c_out, column_tile, out, s);
   }
-  if (path == kNarrow) {
-    if (dtype == TSC_F32)
-      return dispatch_narrow<float>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out,
-                                    k_vol, c_out, out, s);
-    if (dtype == TSC_F16)
-      return dispatch_narrow<__half>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out,
-                                     k_vol, c_out, out, s);
-    return dispatch_narrow<__hip_bfloat16>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered,
-                                           n_out, k_vol, c_out, out, s);
-  }
   if (dtype == TSC_F32)
-    return dispatch_valu<float>(feat, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out, k_vol,
-                                c_out, out, s);
+    return dispatch_narrow<float>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out,
+                                  k_vol, c_out, out, s);
   if (dtype == TSC_F16)
-    return dispatch_valu<__half>(feat, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out, k_vol,
-                                 c_out, out, s);
-  return dispatch_valu<__hip_bfloat16>(feat, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out,
-                                       k_vol, c_out, out, s);
+    return dispatch_narrow<__half>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out,
+                                   k_vol, c_out, out, s);
+  return dispatch_narrow<__hip_bfloat16>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered,
+                                         n_out, k_vol, c_out, out, s);
 }
 
 extern "C" int tsc_conv_forward(const void* feat, int32_t dtype, int64_t n_in, int32_t c_in,
@@ -2010,9 +1957,7 @@ extern "C" const char* tsc_conv_kernel_name(int32_t dtype, int32_t c_in, int32_t
       const MfmaChoice ch = choose_mfma(dtype, c_in, c_out, k_vol, n_out, 0);
       return ch.split ? "conv_split_kernel" : ch.dma ? "conv_dma_kernel" : "conv_mfma_kernel";
     }
-    case kNarrow:
-      return "conv_narrow_kernel";
     default:
-      return "conv_valu_kernel";
+      return "conv_narrow_kernel";
   }
 }
