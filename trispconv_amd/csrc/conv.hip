@@ -244,6 +244,110 @@ template <> struct MfmaOp<float> {
   }
 };
 
+// ------------------------------------------------- f32 on the bf16 cores --
+// f32 operands as sums of three bf16 values each, x = hi + mid + lo: hi is x
+// rounded to bf16, mid the rest rounded to bf16, lo what is left, which has at
+// most 8 significant bits and is exact.  A product is then six bf16 products,
+//   x * y = lo*hi' + hi*lo' + mid*mid' + mid*hi' + hi*mid' + hi*hi'
+// (exact each, summed in the f32 accumulator); the three left out are below
+// 2^-24 of it.  A 32x32x16 bf16 MFMA takes 32 cycles, eight 32x32x2 f32 ones
+// take 512, so a stage's matrix work falls to 6 * 32 / 512 = 0.375 of the f32
+// unit's; the splits are vector work (11 instructions for two values).
+// Relative 2-norm error against 64 bits, the f32 unit's and this one's:
+// 27 x 64 -> 64 SubM, 100k rows, 5.3e-7 and 4.5e-7; 64 -> 64 stride 2 on
+// LiDAR voxels 4.4e-7 and 3.7e-7.  Their times (the first's launch, the
+// second's whole frame with its build and plan): 179 -> 133 us, 301 -> 251 us.
+// A value that is not finite or rounds to infinity in bf16 makes its products
+// NaN; the accumulators that end up not finite are computed once more on the
+// f32 unit (rerun below), so such outputs are what that unit gives.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint32_t& mid,
+                                           uint32_t& lo) {
+  auto pack = [](float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+  };
+  auto low = [](uint32_t v) { return __uint_as_float(v << 16); };
+  auto high = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
+  hi = pack(x, y);
+  const float rx = x - low(hi), ry = y - high(hi);
+  mid = pack(rx, ry);
+  lo = pack(rx - low(mid), ry - high(mid));
+}
+
+struct Split8 {  // eight f32 values of one operand
+  bf16x8 hi, mid, lo;
+};
+__device__ __forceinline__ Split8 split8(const uint4& a, const uint4& b) {
+  const float4 x = __builtin_bit_cast(float4, a), y = __builtin_bit_cast(float4, b);
+  uint4 h, m, l;
+  split_pair(x.x, x.y, h.x, m.x, l.x);
+  split_pair(x.z, x.w, h.y, m.y, l.y);
+  split_pair(y.x, y.y, h.z, m.z, l.z);
+  split_pair(y.z, y.w, h.w, m.w, l.w);
+  return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m),
+          __builtin_bit_cast(bf16x8, l)};
+}
+__device__ __forceinline__ f32x16 mfma_split(const Split8& a, const Split8& b, f32x16 c) {
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.lo, b.hi, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.lo, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.mid, b.mid, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.mid, b.hi, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.mid, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.hi, c, 0, 0, 0);
+}
+
+// A split weight slab in LDS: [plane hi/mid/lo][column block nb][half t of the
+// 32-channel chunk][lane][16 bytes].  Vector u of block nb (four f32 values of
+// each lane, as packed) goes to half u / 2, eight bytes at (u % 2) * 8: an
+// operand of half t is then one 16-byte read per plane.
+template <int NB>
+__device__ __forceinline__ void store_split(uint4* slab, int nb, int u, int lane, const uint4& v) {
+  const float4 x = __builtin_bit_cast(float4, v);
+  uint2 pl[3];
+  split_pair(x.x, x.y, pl[0].x, pl[1].x, pl[2].x);
+  split_pair(x.z, x.w, pl[0].y, pl[1].y, pl[2].y);
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+    reinterpret_cast<uint2*>(slab)[(((p * NB + nb) * 2 + (u >> 1)) * 64 + lane) * 2 + (u & 1)] = pl[p];
+}
+template <int NB>
+__device__ __forceinline__ Split8 load_split(const uint4* slab, int nb, int t, int lane) {
+  auto plane = [&](int p) {
+    return __builtin_bit_cast(bf16x8, slab[((p * NB + nb) * 2 + t) * 64 + lane]);
+  };
+  return {plane(0), plane(1), plane(2)};
+}
+
+// The elements of this lane's accumulators that are not finite, one bit each.
+template <int RB, int NB>
+struct NonFinite {
+  uint32_t bits[(RB * NB + 1) / 2];
+  __device__ __forceinline__ bool any() const {
+    uint32_t m = 0;
+    for (uint32_t b : bits) m |= b;
+    return m != 0;
+  }
+  __device__ __forceinline__ void find(const f32x16 (&acc)[RB][NB]) {
+    for (uint32_t& b : bits) b = 0;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const bool bad = (__float_as_uint(acc[rb][nb][i]) & 0x7f800000u) == 0x7f800000u;
+          const int e = (rb * NB + nb) * 16 + i;
+          bits[e / 32] |= (bad ? 1u : 0u) << (e % 32);
+        }
+  }
+  __device__ __forceinline__ bool has(int rb, int nb, int i) const {
+    const int e = (rb * NB + nb) * 16 + i;
+    return (bits[e / 32] >> (e % 32)) & 1u;
+  }
+};
+
 constexpr int kTileRows = kConvTileRows;  // 4 waves x 64 rows
 constexpr int kSplitRows = 64;            // rows of a small-layer tile (its 4 waves split the slots)
 
@@ -292,7 +396,8 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   constexpr bool FULL = SLAB_VECS % 256 == 0;
   static_assert(WV <= 4, "weight slab too large for the register stage");
 
-  __shared__ __attribute__((aligned(16))) uint4 s_w[2][SLAB_VECS];
+  static_assert(!F32 || (UB == 4 && SLAB_VECS == 256 * NB), "a wave's share is one vector per block");
+  __shared__ __attribute__((aligned(16))) uint4 s_w[2][F32 ? SLAB_VECS * 3 / 2 : SLAB_VECS];
   __shared__ __attribute__((aligned(16))) int32_t s_orow[kTileRows];
   __shared__ float s_bias[BN];        // this column tile's bias in fp32 (0 without one)
   __shared__ float s_scale[BN];       // its affine epilogue (1 and 0 without one)
@@ -432,7 +537,14 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
     if constexpr (WV > 2) w2 = src[512];
     if constexpr (WV > 3) w3 = src[768];
   };
-  auto store_w = [&](uint4* dst) {
+  auto store_w = [&](uint4* dst, auto split) {
+    if constexpr (decltype(split)::value) {  // vector m*256 + t: block m, vector `wave` of it
+      store_split<NB>(dst, 0, wave, lane, w0);
+      if constexpr (WV > 1) store_split<NB>(dst, 1, wave, lane, w1);
+      if constexpr (WV > 2) store_split<NB>(dst, 2, wave, lane, w2);
+      if constexpr (WV > 3) store_split<NB>(dst, 3, wave, lane, w3);
+      return;
+    }
     if (FULL || t < SLAB_VECS) dst[t] = w0;
     if constexpr (WV > 1) dst[256 + t] = w1;
     if constexpr (WV > 2) dst[512 + t] = w2;
@@ -466,9 +578,23 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   // serves the other workgroup's wave on the same SIMD.  Inside a computed
   // stage, rows without input through the slot multiply the zero row and add
   // exact zeros, so skipping a stage leaves every finite result unchanged.
-  auto compute = [&](auto slot, const uint4* sw, int k) {
+  auto compute = [&](auto slot, const uint4* sw, int k, auto split) {
     constexpr int S = decltype(slot)::value;
     if (k >= K || !((wmask >> k) & 1)) return;
+    if constexpr (decltype(split)::value) {
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        const Split8 a0 = split8(ring[S][0][2 * t2], ring[S][0][2 * t2 + 1]);
+        const Split8 a1 = split8(ring[S][1][2 * t2], ring[S][1][2 * t2 + 1]);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const Split8 b = load_split<NB>(sw, nb, t2, lane);
+          acc[0][nb] = mfma_split(a0, b, acc[0][nb]);
+          acc[1][nb] = mfma_split(a1, b, acc[1][nb]);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < UB; ++u) {
 #pragma unroll
@@ -496,37 +622,45 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
     }
   };
 
-  // current stage (kc, cc) and the next one (kn, cn)
-  int kc = -1, cc = nch - 1;
-  advance(kc, cc);  // the tile's first slot
-  int kn = kc, cn = cc;
-  advance(kn, cn);
-  load_w(kc, cc);
-  load_a(Slot<0>{}, kc, cc);
-  store_w(s_w[0]);
-  __syncthreads();
-
   // Two waves per SIMD (two workgroups per CU): while one wave waits for its
   // gathers or at the barrier, the other's MFMAs keep the matrix core busy.
   // The next stage's loads are issued before this stage's MFMAs, the weights
   // first (they are waited for before the barrier, the gathered operands only
   // in the next stage); the scheduling barrier keeps the compiler from sinking
   // the loads below the MFMAs.
-  auto body = [&](auto slot) {
-    constexpr int S = decltype(slot)::value;
-    load_w(kn, cn);                           // next stage's weights
-    load_a(Slot<(S + 1) % RING>{}, kn, cn);   // next stage's operands
-    __builtin_amdgcn_sched_barrier(0);
-    compute(Slot<S>{}, s_w[S], kc);
-    store_w(s_w[(S + 1) % RING]);
-    __syncthreads();
-    kc = kn;
-    cc = cn;
+  auto run = [&](auto split) {
+    // current stage (kc, cc) and the next one (kn, cn)
+    int kc = -1, cc = nch - 1;
+    advance(kc, cc);  // the tile's first slot
+    int kn = kc, cn = cc;
     advance(kn, cn);
+    load_w(kc, cc);
+    load_a(Slot<0>{}, kc, cc);
+    store_w(s_w[0], split);
+    __syncthreads();
+    auto body = [&](auto slot) {
+      constexpr int S = decltype(slot)::value;
+      load_w(kn, cn);                           // next stage's weights
+      load_a(Slot<(S + 1) % RING>{}, kn, cn);   // next stage's operands
+      __builtin_amdgcn_sched_barrier(0);
+      compute(Slot<S>{}, s_w[S], kc, split);
+      store_w(s_w[(S + 1) % RING], split);
+      __syncthreads();
+      kc = kn;
+      cc = cn;
+      advance(kn, cn);
+    };
+    while (kc < K) {
+      body(Slot<0>{});
+      body(Slot<1>{});
+    }
   };
-  while (kc < K) {
-    body(Slot<0>{});
-    body(Slot<1>{});
+  run(std::bool_constant<F32>{});
+  NonFinite<2, NB> bad;
+  bool rerun = false;
+  if constexpr (F32) {
+    bad.find(acc);
+    rerun = __syncthreads_or(bad.any());
   }
 
   // ---- epilogue: + bias (and the affine map and ReLU when asked), round
@@ -590,6 +724,35 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
         *reinterpret_cast<uint4*>(out + (int64_t)orows[q] * c_out + nbt * BN + ch * (16 / (int)sizeof(T))) = vals[q];
     }
   }
+  if constexpr (F32) {
+    if (rerun) {  // workgroup-uniform, and rare
+      // the stores above are done, and the staged slot lists are read again
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      for (int k = 0; k < K; ++k) {
+        const int32_t o = s_orow[t];
+        const int64_t col = nbr_ordered ? tile0 + t : (int64_t)o;
+        s_nbr[k * kTileRows + t] = o < 0 ? -1 : nbr ? nbr[(int64_t)k * n_out + col] : o;
+      }
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[rb][nb] = f32x16{};
+      __syncthreads();
+      run(std::false_type{});
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int32_t o = s_orow[wave * 64 + rb * 32 + (i >> 2) * 8 + h * 4 + (i & 3)];
+            if (bad.has(rb, nb, i) && o >= 0)
+              out[(int64_t)o * c_out + nbt * BN + nb * 32 + (lane & 31)] = from_f32<T>(
+                  finish(acc[rb][nb][i] + cbias[nb], cscale[nb], cshift[nb], affine, relu));
+          }
+    }
+  }
 }
 
 // ------------------------------------------------------ LDS DMA variant --
@@ -627,9 +790,10 @@ __device__ __forceinline__ void dma_b32(const void* g, uint32_t m0) {
 
 // Dynamic LDS of conv_dma_kernel: two weight slabs, each wave's operand rows
 // of one stage (32 * RB rows x 128 bytes) and two stages of its map entries.
+// f32: one weight slab as loaded and two split ones.
 template <typename T, int BN, int RB>
 constexpr size_t dma_pool_bytes() {
-  return (size_t)2 * BN * 128 + (size_t)4 * 32 * RB * 128 + (size_t)4 * 2 * 256;
+  return (size_t)(sizeof(T) == 4 ? 4 : 2) * BN * 128 + (size_t)4 * 32 * RB * 128 + (size_t)4 * 2 * 256;
 }
 
 template <typename T, int BN, int RB>
@@ -651,10 +815,16 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   constexpr int TR = 4 * WR;                 // rows of a tile
   constexpr int A_BYTES = WR * CK * (int)sizeof(T);  // one wave's rows of one stage (4 or 8 KB)
   static_assert(RB == 1 || RB == 2, "one or two 32-row blocks per wave");
-  static_assert(A_BYTES == 4096 * RB && (size_t)2 * SLAB_BYTES + 4 * A_BYTES + 2048 == dma_pool_bytes<T, BN, RB>(),
+  // f32 slabs are loaded into one buffer, of which each wave loads and then
+  // reads only its own vectors, and split into two others that all waves read
+  constexpr int SPLIT_BYTES = SLAB_BYTES * 3 / 2;
+  constexpr int W_BYTES = F32 ? SLAB_BYTES + 2 * SPLIT_BYTES : 2 * SLAB_BYTES;
+  static_assert(!F32 || WD == NB, "a wave's share of an f32 slab is one vector per column block");
+  static_assert(A_BYTES == 4096 * RB && (size_t)W_BYTES + 4 * A_BYTES + 2048 == dma_pool_bytes<T, BN, RB>(),
                 "pool layout");
-  // pool: slabs [2][SLAB_BYTES] | operand rows [4 waves][A_BYTES] |
-  // map entries [4 waves][2][64]; the output staging at the end
+  // pool: slabs [W_BYTES] (f16/bf16 two; f32 one, then two split) | operand
+  // rows [4 waves][A_BYTES] | map entries [4 waves][2][64]; the output staging
+  // at the end
   extern __shared__ __attribute__((aligned(16))) char pool[];
   __shared__ __attribute__((aligned(16))) int32_t s_orow[TR];
   __shared__ float s_bias[BN];
@@ -780,11 +950,12 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
 
   // LDS offsets for M0 (wave-uniform) and the same places as pointers
   const uint32_t w_lds = lds_offset(pool);                                   // slab P: + P * SLAB_BYTES
-  const uint32_t a_lds = w_lds + 2 * SLAB_BYTES + wave_u * A_BYTES;
-  const uint32_t e_lds = w_lds + 2 * SLAB_BYTES + 4 * A_BYTES + wave_u * 512;  // entries P: + P * 256
+  const uint32_t a_lds = w_lds + W_BYTES + wave_u * A_BYTES;
+  const uint32_t e_lds = w_lds + W_BYTES + 4 * A_BYTES + wave_u * 512;  // entries P: + P * 256
   const uint4* s_w = reinterpret_cast<const uint4*>(pool);
-  const char* s_a = pool + 2 * SLAB_BYTES + wave * A_BYTES;
-  const int32_t* s_e = reinterpret_cast<const int32_t*>(pool + 2 * SLAB_BYTES + 4 * A_BYTES + wave * 512);
+  uint4* s_split = reinterpret_cast<uint4*>(pool + SLAB_BYTES);  // f32: split slab P: + P * SPLIT_BYTES
+  const char* s_a = pool + W_BYTES + wave * A_BYTES;
+  const int32_t* s_e = reinterpret_cast<const int32_t*>(pool + W_BYTES + 4 * A_BYTES + wave * 512);
 
   // Map entries: lane l < WR loads the entry of its wave's row l (lanes
   // past WR load -1 from the no-row array).  Operand rows:
@@ -804,6 +975,13 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
 #pragma unroll
     for (int m = 0; m < WD; ++m)
       dma_b128(src + m * 256, w_lds + P * SLAB_BYTES + (m * 256 + wave_u * 64) * 16);
+  };
+  // f32: this wave's vectors of the loaded slab (block m, vector `wave`), as
+  // three bf16 planes, into split slab P
+  auto split_slab = [&](int P) {
+#pragma unroll
+    for (int m = 0; m < NB; ++m)
+      store_split<NB>(s_split + P * (SPLIT_BYTES / 16), m, wave, lane, s_w[m * 256 + t]);
   };
   // DMA addresses.  A present row's is one 64-bit multiply-add (row times
   // row bytes plus the lane's base), an absent row's the zero row, chosen by a
@@ -868,23 +1046,6 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[rb][nb][i] = 0.f;
 
-  // stages s (kc, cc), s + 1 (kn, cn) and s + 2 (kp, cp)
-  int kc = -1, cc = nch - 1;
-  advance(kc, cc);
-  int kn = kc, cn = cc;
-  advance(kn, cn);
-  int kp = kn, cp = cn;
-  advance(kp, cp);
-  if (kc < K) {
-    dma_entries(0, kc);
-    dma_slab(0, kc, cc);
-  }
-  if (kn < K) dma_entries(1, kn);
-  wait_vm0();
-  dma_rows(0, cc, blocks(kc));
-  wait_vm0();
-  __syncthreads();
-
   // Stage s (slab and entry buffers S = s % 2), with the three waits:
   //  1. vmcnt(0): this wave's rows of s have landed (issued in stage s - 1);
   //  2. the slab of s + 1 and the entries of s + 2 go out; the rows of s and
@@ -893,70 +1054,123 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   //  3. MFMAs of s; vmcnt(4 * RB) (or 0 when no rows went out): the slab and
   //     the entries have landed, the 4 * RB row loads of s + 1 may still be in
   //     flight; the barrier then publishes the slab to every wave.
-  auto body = [&](auto slot) {
-    constexpr int S = decltype(slot)::value;
-    wait_vm0();
-    if (kn < K) dma_slab(S ^ 1, kn, cn);
-    if (kp < K) dma_entries(S, kp);
-    const int cur = blocks(kc);
-    uint4 a[RB][UB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      if ((cur >> rb) & 1) {
-#pragma unroll
-        for (int u = 0; u < UB; ++u) a[rb][u] = a_read(rb, u);
-      }
+  // f32 (split): the slab of s + 1 lands in the one load buffer, whose vectors
+  // each wave splits into split slab S ^ 1 between wait 3 and the barrier; the
+  // wait in 2 also covers those reads, so the slab of s + 2 may land there.
+  auto run = [&](auto split) {
+    constexpr bool SPLIT = decltype(split)::value;
+    // stages s (kc, cc), s + 1 (kn, cn) and s + 2 (kp, cp)
+    int kc = -1, cc = nch - 1;
+    advance(kc, cc);
+    int kn = kc, cn = cc;
+    advance(kn, cn);
+    int kp = kn, cp = cn;
+    advance(kp, cp);
+    if (kc < K) {
+      dma_entries(0, kc);
+      dma_slab(0, kc, cc);
     }
-    wait_lgkm0();
-    const int nxt = blocks(kn);
-    dma_rows(S ^ 1, cn, nxt);
-    // the MFMAs of the blocks that use slot kc (a wave-uniform branch per
-    // block; one loop, so the register allocation is that of a full wave)
-    if (cur) {
-      const uint4* sw = s_w + S * SLAB_VECS;
+    if (kn < K) dma_entries(1, kn);
+    wait_vm0();
+    if constexpr (SPLIT) {
+      if (kc < K) split_slab(0);
+      wait_lgkm0();
+    }
+    dma_rows(0, cc, blocks(kc));
+    wait_vm0();
+    __syncthreads();
+
+    auto body = [&](auto slot) {
+      constexpr int S = decltype(slot)::value;
+      wait_vm0();
+      if (kn < K) dma_slab(SPLIT ? 0 : S ^ 1, kn, cn);
+      if (kp < K) dma_entries(S, kp);
+      const int cur = blocks(kc);
+      uint4 a[RB][UB];
 #pragma unroll
-      for (int u = 0; u < UB; ++u) {
+      for (int rb = 0; rb < RB; ++rb) {
+        if ((cur >> rb) & 1) {
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const uint4 bv = sw[(nb * UB + u) * 64 + lane];
-          if constexpr (F32) {
-            // four 32x32x2 steps per vector: step e uses element e of A and B
-            const float4 b4 = __builtin_bit_cast(float4, bv);
-            const float bs[4] = {b4.x, b4.y, b4.z, b4.w};
+          for (int u = 0; u < UB; ++u) a[rb][u] = a_read(rb, u);
+        }
+      }
+      wait_lgkm0();
+      const int nxt = blocks(kn);
+      dma_rows(S ^ 1, cn, nxt);
+      // the MFMAs of the blocks that use slot kc (a wave-uniform branch per
+      // block; one loop, so the register allocation is that of a full wave)
+      if (SPLIT && cur) {
+        const uint4* sw = s_split + S * (SPLIT_BYTES / 16);
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+        for (int t2 = 0; t2 < 2; ++t2) {
+          Split8 as[RB];
 #pragma unroll
-              for (int rb = 0; rb < RB; ++rb) {
-                if ((cur >> rb) & 1) {
-                  const float4 a4 = __builtin_bit_cast(float4, a[rb][u]);
-                  const float as[4] = {a4.x, a4.y, a4.z, a4.w};
-                  acc[rb][nb] = Op::run(as[e], bs[e], acc[rb][nb]);
-                }
-              }
-          } else {
-            const V b = __builtin_bit_cast(V, bv);
+          for (int rb = 0; rb < RB; ++rb)
+            if ((cur >> rb) & 1) as[rb] = split8(a[rb][2 * t2], a[rb][2 * t2 + 1]);
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            const Split8 b = load_split<NB>(sw, nb, t2, lane);
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
-              if ((cur >> rb) & 1)
-                acc[rb][nb] = Op::run(__builtin_bit_cast(V, a[rb][u]), b, acc[rb][nb]);
+              if ((cur >> rb) & 1) acc[rb][nb] = mfma_split(as[rb], b, acc[rb][nb]);
+          }
+        }
+      } else if (cur) {
+        const uint4* sw = s_w + S * SLAB_VECS;
+#pragma unroll
+        for (int u = 0; u < UB; ++u) {
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            const uint4 bv = sw[(nb * UB + u) * 64 + lane];
+            if constexpr (F32) {
+              // four 32x32x2 steps per vector: step e uses element e of A and B
+              const float4 b4 = __builtin_bit_cast(float4, bv);
+              const float bs[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) {
+                  if ((cur >> rb) & 1) {
+                    const float4 a4 = __builtin_bit_cast(float4, a[rb][u]);
+                    const float as[4] = {a4.x, a4.y, a4.z, a4.w};
+                    acc[rb][nb] = Op::run(as[e], bs[e], acc[rb][nb]);
+                  }
+                }
+            } else {
+              const V b = __builtin_bit_cast(V, bv);
+#pragma unroll
+              for (int rb = 0; rb < RB; ++rb)
+                if ((cur >> rb) & 1)
+                  acc[rb][nb] = Op::run(__builtin_bit_cast(V, a[rb][u]), b, acc[rb][nb]);
+            }
           }
         }
       }
+      wait_rows(__builtin_popcount(nxt));
+      if constexpr (SPLIT) {
+        if (kn < K) split_slab(S ^ 1);
+      }
+      __syncthreads();
+      kc = kn;
+      cc = cn;
+      kn = kp;
+      cn = cp;
+      advance(kp, cp);
+    };
+    while (kc < K) {
+      body(Slot<0>{});
+      body(Slot<1>{});
     }
-    wait_rows(__builtin_popcount(nxt));
+    wait_vm0();
     __syncthreads();
-    kc = kn;
-    cc = cn;
-    kn = kp;
-    cn = cp;
-    advance(kp, cp);
   };
-  while (kc < K) {
-    body(Slot<0>{});
-    body(Slot<1>{});
+  run(std::bool_constant<F32>{});
+  NonFinite<RB, NB> bad;
+  bool rerun = false;
+  if constexpr (F32) {
+    bad.find(acc);
+    rerun = __syncthreads_or(bad.any());
   }
-  wait_vm0();
-  __syncthreads();
 
   // ---- epilogue, as in conv_mfma_kernel, staged in the pool
   const bool affine = ep.mean != nullptr;
@@ -1013,6 +1227,28 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
       if (orows[qq] >= 0)
         store_out(out + (int64_t)orows[qq] * c_out + nbt * BN + ch * (16 / (int)sizeof(T)), vals[qq],
                   whole_lines);
+    }
+  }
+  if constexpr (F32) {
+    if (rerun) {  // workgroup-uniform, and rare
+      wait_vm0();  // the stores above are done
+      __syncthreads();
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[rb][nb] = f32x16{};
+      run(std::false_type{});
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int32_t o = s_orow[wave * WR + rb * 32 + (i >> 2) * 8 + h * 4 + (i & 3)];
+            if (bad.has(rb, nb, i) && o >= 0)
+              out[(int64_t)o * c_out + nbt * BN + nb * 32 + (lane & 31)] = from_f32<T>(
+                  finish(acc[rb][nb][i] + cbias[nb], cscale[nb], cshift[nb], affine, relu));
+          }
     }
   }
 }
@@ -1605,6 +1841,10 @@ int launch_mfma(const void* feat, int c_in, const void* W, const Epilogue& ep,
   const int row_bytes = BN * (int)sizeof(T);
   const size_t lds_out = (size_t)4 * mfma_stage_rows(row_bytes) * (row_bytes + 16);  // 4 waves
   const size_t lds = lds_nbr > lds_out ? lds_nbr : lds_out;
+  // with the weight slabs it may pass 64 KB (K <= 64 slots)
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&conv_mfma_kernel<T, BN, CK>),
+                                 64 * kTileRows * (int)sizeof(int32_t)))
+    return rc;
   conv_mfma_kernel<T, BN, CK><<<grid, 256, lds, s>>>(
       static_cast<const T*>(feat), c_in, static_cast<const T*>(W), ep, nbr, order,
       nbr_ordered, n_out, K, c_out, static_cast<T*>(out));
@@ -1691,6 +1931,7 @@ MfmaChoice choose_mfma(int dtype, int c_in, int c_out, int K, int64_t n_out, int
     c.bn = column_tile;
     return c;
   }
+  if (dtype == TSC_F32 && c.bn > 64) c.bn = 64;  // split slabs of 128 columns leave one workgroup per CU
   while (c.bn > 32 && ceil_div(n_out, kTileRows) * (c_out / c.bn) < 512) c.bn /= 2;
   c.split = c.bn == 32 && K >= 8 && ceil_div(n_out, kTileRows) * (c_out / c.bn) < 128;
   c.dma = !c.split && K > 1 && c.ck * dtype_bytes(dtype) == 128 && c_in % c.ck == 0;
