@@ -324,10 +324,16 @@ __device__ __forceinline__ Split8 load_split(const uint4* slab, int nb, int t, i
 template <int RB, int NB>
 struct NonFinite {
   uint32_t bits[(RB * NB + 1) / 2];
-  __device__ __forceinline__ bool any() const {
-    uint32_t m = 0;
-    for (uint32_t b : bits) m |= b;
-    return m != 0;
+  // whether there are any: 0 * x is 0 for every finite x, else NaN
+  static __device__ __forceinline__ bool any(const f32x16 (&acc)[RB][NB]) {
+    float z = 0.f;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) z = fmaf(acc[rb][nb][i], 0.f, z);
+    return !(z == 0.f);
   }
   __device__ __forceinline__ void find(const f32x16 (&acc)[RB][NB]) {
     for (uint32_t& b : bits) b = 0;
@@ -656,12 +662,8 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
     }
   };
   run(std::bool_constant<F32>{});
-  NonFinite<2, NB> bad;
   bool rerun = false;
-  if constexpr (F32) {
-    bad.find(acc);
-    rerun = __syncthreads_or(bad.any());
-  }
+  if constexpr (F32) rerun = __syncthreads_or(NonFinite<2, NB>::any(acc));
 
   // ---- epilogue: + bias (and the affine map and ReLU when asked), round
   // once, store each output element once.
@@ -726,6 +728,8 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   }
   if constexpr (F32) {
     if (rerun) {  // workgroup-uniform, and rare
+      NonFinite<2, NB> bad;
+      bad.find(acc);
       // the stores above are done, and the staged slot lists are read again
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -1165,12 +1169,8 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
     __syncthreads();
   };
   run(std::bool_constant<F32>{});
-  NonFinite<RB, NB> bad;
   bool rerun = false;
-  if constexpr (F32) {
-    bad.find(acc);
-    rerun = __syncthreads_or(bad.any());
-  }
+  if constexpr (F32) rerun = __syncthreads_or(NonFinite<RB, NB>::any(acc));
 
   // ---- epilogue, as in conv_mfma_kernel, staged in the pool
   const bool affine = ep.mean != nullptr;
@@ -1231,6 +1231,8 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   }
   if constexpr (F32) {
     if (rerun) {  // workgroup-uniform, and rare
+      NonFinite<RB, NB> bad;
+      bad.find(acc);
       wait_vm0();  // the stores above are done
       __syncthreads();
 #pragma unroll
@@ -1900,52 +1902,90 @@ struct MfmaChoice {
   int rb;      // its 32-row blocks per wave (tiles of 128 * rb rows)
 };
 
-// Layers with fewer 256-row tiles than this run the direct-to-LDS kernel on
-// 128-row tiles (32 rows per wave).  On such layers the kernel lasts as long
-// as its heaviest tiles' chain of stages (27 slots x the channel chunks, each
-// stage's MFMAs shared by the waves on a SIMD); halving a wave's rows halves
-// the MFMAs of each stage and, with the smaller LDS pool, lets up to four
-// workgroups share a CU.  Measured: the 166k-row 64->64 fp32 strided layer
-// (651 tiles) 182 -> 140-152 us, the 32k-row 64->64 fp16 layers 31.4 -> 30.1
-// us; the 500k-row 128->128 fp16 layer (1954 tiles) is slower that way, 327
-// -> 339 us, where two 64-row waves share each weight slab read from LDS.
+// Layers of at least this many 256-row tiles always run the direct-to-LDS
+// kernel at 64 rows per wave: the sum of all tiles' work bounds them, and two
+// 64-row waves share each weight slab read from LDS (the 500k-row 128->128
+// fp16 layer, 1954 tiles: 327 us, 339 us at 32 rows per wave).
 constexpr int64_t kShortTiles = 1024;
+constexpr int64_t kCus = 256;
 
-// Narrower column tiles for small layers: below two workgroups per CU, halve
-// BN (each halving doubles the workgroups; gathers repeat per column tile,
-// which a small layer can afford).  Layers that would leave more than half
-// the CUs without a 256-row workgroup run on 64-row tiles with the slots
-// split over the waves (the narrowing has then always reached 32 columns).
-// Measured on 64->64 fp16 SubM layers: 9.7k rows (76 workgroups) 28.8 ->
-// 20.0 us, but 32k rows (252 workgroups) 30.7 -> 38 us, where the four waves'
-// separate weight loads cost more than the shorter slot chain saves.  Short
-// slot lists (K < 8) gain nothing from splitting.  column_tile != 0 forces
-// the 256-row kernel with that width (every width sums each output in the
-// same order, so all give the same bits), always on the register-gather
-// kernel.  The 256-row kernel's direct-to-LDS variant serves layers whose
-// stages are 128 bytes of each row (f16/bf16 with C_in % 64 == 0, f32 with
-// C_in % 32 == 0) and that have a map (K > 1); it sums in the same order too.
-MfmaChoice choose_mfma(int dtype, int c_in, int c_out, int K, int64_t n_out, int column_tile) {
+// Workgroups of the direct-to-LDS kernel a CU's 160 KB of LDS hold (its pool
+// and up to 3 KB of static arrays).
+int dma_per_cu(int dtype, int bn, int rb) {
+  return 163840 / ((dtype == TSC_F32 ? 4 : 2) * bn * 128 + 16384 * rb + 2048 + 3072);
+}
+
+// Column tile width, kernel and rows per wave of a 32x32-tile layer.  Below a
+// few workgroups per CU a layer's time is one tile's chain of stages (27 slots
+// x the channel chunks), which a narrower or shorter tile shortens, against
+// repeated gathers per column tile; the lines are where the two meet, from a
+// sweep of every width and row count over layers of 16-768 channels and 3k-400k
+// rows, all dtypes.  Times in us are of one launch from a captured graph.
+//   * Column tile.  The widest that leaves enough tiles: direct-to-LDS f16/bf16
+//     128-row tiles, 400 at 128 columns and 180 at 64; f32 512 at 64 (its
+//     stages are longer); other layers 256-row tiles, 360 at 128 columns and
+//     128 at 64 (300 for f32 and for K < 12).  64->64 fp16: 120k rows 59 -> 41
+//     with 64 columns for 32, 16k rows 18.7 with 64 and 16.2 with 32; 128->128
+//     fp16: 70k rows 96 at 64 and 89 at 128, 40k rows 56 and 59; 192->192, 40k
+//     rows 142 -> 107; 64->64 f32: 70k rows 138 -> 118, 40k rows 88 at 64 and
+//     79 at 32.  Short slot lists (K < 8) keep the line at 512 256-row tiles.
+//   * Slot split (conv_split_kernel, 64-row tiles of 32 columns, K >= 8) up to
+//     one tile per CU for f16/bf16 layers the direct-to-LDS kernel takes
+//     (64->64, 8k rows 14.1 against 15.7; 10k rows 18.5 against 15.9), two for
+//     a single column tile (inverse 64->32, 30k rows 15.2 against 17.1), for
+//     K < 12 (32->64 with 8 slots, 20k rows 10.2 against 8.6) and for f32
+//     (64->64, 16k rows 48 against 50; 128->128, 16k rows 173 against 115), and
+//     two and a half for the other f16/bf16 layers (32->32, 28k rows 12.8
+//     against 15.7; 48->64, 20k rows 20.2 against 24.3, 28k 25.1 against 24.5).
+//   * Rows per wave of the direct-to-LDS kernel: 32 (128-row tiles) below
+//     kShortTiles 256-row tiles, as halving a wave's rows halves each stage's
+//     MFMAs and the smaller pool lets more workgroups share a CU; but 64 where
+//     256-row tiles fit the chip at once and 128-row ones do not (128->128
+//     fp16, 120k rows: 106 -> 91; 256->256 bf16, 60k: 207 -> 162; 64->64 f32,
+//     120k: 149 -> 132).  Not with fewer input than output rows: an inverse
+//     layer's tiles use from one slot to eight, and its launch lasts as long
+//     as the chain of those with eight (768->256, 60k rows: 142 against 180).
+// column_tile != 0 forces the 256-row register-gather kernel with that width.
+// Every width and both 256-row kernels sum each output in the same order, so
+// all give the same bits.  The direct-to-LDS kernel serves layers whose stages
+// are 128 bytes of each row (f16/bf16 with C_in % 64 == 0, f32 with C_in % 32
+// == 0) and that have a map (K > 1).
+MfmaChoice choose_mfma(int dtype, int c_in, int c_out, int K, int64_t n_in, int64_t n_out,
+                       int column_tile) {
   MfmaChoice c{pick_bn(c_out), pick_ck(dtype, c_in), false, false, 2};
   if (column_tile) {
     c.bn = column_tile;
     return c;
   }
-  if (dtype == TSC_F32 && c.bn > 64) c.bn = 64;  // split slabs of 128 columns leave one workgroup per CU
-  while (c.bn > 32 && ceil_div(n_out, kTileRows) * (c_out / c.bn) < 512) c.bn /= 2;
-  c.split = c.bn == 32 && K >= 8 && ceil_div(n_out, kTileRows) * (c_out / c.bn) < 128;
-  c.dma = !c.split && K > 1 && c.ck * dtype_bytes(dtype) == 128 && c_in % c.ck == 0;
-  if (c.dma && ceil_div(n_out, kTileRows) * (c_out / c.bn) < kShortTiles) c.rb = 1;
+  const bool f32 = dtype == TSC_F32;
+  if (f32 && c.bn > 64) c.bn = 64;  // split slabs of 128 columns leave one workgroup per CU
+  const bool dma = K > 1 && c.ck * dtype_bytes(dtype) == 128 && c_in % c.ck == 0;
+  auto tiles = [&](int rows) { return ceil_div(n_out, rows) * (c_out / c.bn); };
+  auto few = [&] {
+    if (K < 8) return tiles(256) < 512;
+    if (dma) return tiles(128) < (f32 ? 512 : c.bn == 128 ? 400 : 180);
+    return tiles(256) < (c.bn == 128 ? 360 : f32 || K < 12 ? 300 : 128);
+  };
+  while (c.bn > 32 && few()) c.bn /= 2;
+  const bool two = f32 || (dma ? c_out == 32 : K < 12);
+  const int64_t split_tiles = two ? 2 * kCus : dma ? kCus : 5 * kCus / 2;
+  c.split = c.bn == 32 && K >= 8 && tiles(kSplitRows) <= split_tiles;
+  c.dma = dma && !c.split;
+  if (c.dma && tiles(256) < kShortTiles) {
+    const bool one_round = tiles(256) <= kCus * dma_per_cu(dtype, c.bn, 2) &&
+                           tiles(128) > kCus * dma_per_cu(dtype, c.bn, 1);
+    c.rb = n_in >= n_out && one_round ? 2 : 1;
+  }
   return c;
 }
 
 template <typename T>
-int dispatch_mfma(const void* feat, int c_in, const void* W, const Epilogue& ep,
+int dispatch_mfma(const void* feat, int64_t n_in, int c_in, const void* W, const Epilogue& ep,
                   const int32_t* nbr, const int32_t* order, int nbr_ordered, int64_t n_out, int K,
                   int c_out, int column_tile, void* out, hipStream_t s) {
   constexpr int dt = std::is_same<T, float>::value ? TSC_F32
                      : std::is_same<T, __half>::value ? TSC_F16 : TSC_BF16;
-  const MfmaChoice ch = choose_mfma(dt, c_in, c_out, K, n_out, column_tile);
+  const MfmaChoice ch = choose_mfma(dt, c_in, c_out, K, n_in, n_out, column_tile);
 #define TSC_MFMA_CASE(BN_, CK_)                                                              \
   if (ch.bn == BN_ && ch.ck == CK_) {                                                        \
     if constexpr (BN_ == 32)                                                                 \
@@ -2138,12 +2178,12 @@ static int conv_forward(const void* feat, int32_t dtype, int64_t n_in, int32_t c
                     (reinterpret_cast<uintptr_t>(out) & 15) == 0,
                 "conv: feature, weight and output buffers must be 16-byte aligned");
     if (dtype == TSC_F32)
-      return dispatch_mfma<float>(feat, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out, k_vol,
+      return dispatch_mfma<float>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out, k_vol,
                                   c_out, column_tile, out, s);
     if (dtype == TSC_F16)
-      return dispatch_mfma<__half>(feat, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out, k_vol,
+      return dispatch_mfma<__half>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out, k_vol,
                                    c_out, column_tile, out, s);
-    return dispatch_mfma<__hip_bfloat16>(feat, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out,
+    return dispatch_mfma<__hip_bfloat16>(feat, n_in, c_in, packed_w, ep, nbr, order, nbr_ordered, n_out,
                                          k_vol, c_out, column_tile, out, s);
   }
   if (dtype == TSC_F32)
@@ -2195,7 +2235,7 @@ extern "C" const char* tsc_conv_kernel_name(int32_t dtype, int32_t c_in, int32_t
   if (!dtype_ok(dtype) || c_in <= 0 || c_out <= 0 || k_vol <= 0 || n_out < 0) return "";
   switch (pick_path(dtype, c_in, c_out, k_vol)) {
     case kMfma: {
-      const MfmaChoice ch = choose_mfma(dtype, c_in, c_out, k_vol, n_out, 0);
+      const MfmaChoice ch = choose_mfma(dtype, c_in, c_out, k_vol, n_out, n_out, 0);
       return ch.split ? "conv_split_kernel" : ch.dma ? "conv_dma_kernel" : "conv_mfma_kernel";
     }
     default:
