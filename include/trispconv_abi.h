@@ -181,6 +181,12 @@ TSC_API int64_t tsc_pairs_from_map_workspace_bytes(int64_t n, int32_t k_vol);
 TSC_API int tsc_pairs_from_map(const int32_t* nbr, int64_t n, int32_t k_vol, int64_t cap,
                                void* ws, int64_t ws_bytes, int32_t* pairs_in,
                                int32_t* pairs_out, tsc_stream_t stream);
+/* The reference's int64 lists from padded tables [K][cap]: the first sizes[k]
+ * (0..cap) entries of every slot k, one slot after the other, in pairs_in and
+ * pairs_out order.  lists_in and lists_out hold the sum of the sizes. */
+TSC_API int tsc_pair_lists(const int32_t* pairs_in, const int32_t* pairs_out, int32_t k_vol,
+                           int64_t cap, const int64_t* sizes /* host, [K] */, int64_t* lists_in,
+                           int64_t* lists_out, tsc_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Strided pairs.  Replaces generate_strided_indice_pairs

@@ -200,8 +200,7 @@ class IndiceData:
 
     def _get_pairs_in(self) -> List[torch.Tensor]:
         if self._pairs_in is None:
-            self._ensure_tables()
-            self._pairs_in = self._slot_views(self._pin)
+            self._make_lists()
         return self._pairs_in
 
     def _set_pairs_in(self, value: List[torch.Tensor]) -> None:
@@ -212,8 +211,7 @@ class IndiceData:
 
     def _get_pairs_out(self) -> List[torch.Tensor]:
         if self._pairs_out is None:
-            self._ensure_tables()
-            self._pairs_out = self._slot_views(self._pout)
+            self._make_lists()
         return self._pairs_out
 
     def _set_pairs_out(self, value: List[torch.Tensor]) -> None:
@@ -222,11 +220,26 @@ class IndiceData:
         self._pairs_out = value
         self._drop_tables()
 
-    def _slot_views(self, table: Optional[torch.Tensor]) -> List[torch.Tensor]:
-        if table is None:
+    def _make_lists(self) -> None:
+        """The reference's int64 lists from the device tables (a list the user
+        assigned stays), all slots of both in one launch."""
+        self._ensure_tables()
+        pin, pout = self._pin, self._pout
+        if pin is None or pout is None:
             raise RuntimeError("IndiceData has neither pair lists nor device tables")
-        counts = [int(c) for c in self.pair_num.tolist()]
-        return [table[k, :c].long() for k, c in enumerate(counts)]
+        K, cap = pin.shape
+        # counts the user assigned may name fewer slots or more entries than a
+        # table has: as slices of it would
+        counts = [len(range(*slice(int(c)).indices(cap))) for c in self.pair_num.tolist()[:K]]
+        sizes = (ctypes.c_int64 * K)(*counts)
+        flat = torch.empty((2, sum(counts)), dtype=torch.int64, device=pin.device)
+        L.check(L.lib().tsc_pair_lists(pin.data_ptr(), pout.data_ptr(), K, cap, sizes,
+                                       flat[0].data_ptr(), flat[1].data_ptr(), L.stream_of(pin)),
+                "pair lists")
+        if self._pairs_in is None:
+            self._pairs_in = list(flat[0].split(counts))
+        if self._pairs_out is None:
+            self._pairs_out = list(flat[1].split(counts))
 
     def _ensure_tables(self) -> None:
         """Padded pair tables from the builder's map (made on first use: the
@@ -244,7 +257,6 @@ class IndiceData:
                                        ws.numel(), pin.data_ptr(), pout.data_ptr(),
                                        L.stream_of(nbr)), "pair lists")
         self._pin, self._pout = pin, pout
-        self._cnt = self.pair_num.to(device=nbr.device, dtype=torch.int32)
 
     def _drop_tables(self) -> None:
         self._pin = self._pout = self._cnt = self._nbr = self._order = None
@@ -875,6 +887,8 @@ def generate_inverse_indice_pairs(fwd: IndiceData) -> IndiceData:
     dev = fwd._pin.device
     K = fwd.K
     cap = fwd._pin.shape[1]
+    if fwd._cnt is None:
+        fwd._cnt = fwd.pair_num.to(device=dev, dtype=torch.int32)
     n_in = len(fwd.input_indices)
     lib = L.lib()
     stream = L.stream_of(fwd._pin)
