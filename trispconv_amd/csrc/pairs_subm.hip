@@ -888,6 +888,124 @@ __global__ void __launch_bounds__(256) subm_probe_333_kernel(
   }
 }
 
+// Kernels 5 cells wide with dil.x == 1 and at most kProbe5Slots slots (5x5x5,
+// a point-cloud network's first layer), for grids of fewer than 2^29 rows: the
+// 3x3x3 form's row lookup, for any number of kernel rows.  A row's five cells
+// lie in two consecutive bitmap words, whose funnel shift gives their
+// occupancy; the row's hits have consecutive ranks, the first hit's as there.
+// Each slot's column entry is one load at (first rank + hits below it), which
+// a row none of whose lanes has a hit skips (a surface's 5x5x5 neighbourhood
+// fills about a quarter of its slots, in few of its rows).  The slot-by-slot
+// probe spends two loads, a bounds test and a cell key on each of 125 slots:
+// 80k surface voxels in 160^3, 69 -> 24 us.
+constexpr int kProbe5Slots = 128;
+
+template <bool TOUCHED>
+__global__ void __launch_bounds__(256) subm_probe_5wide_kernel(
+    int64_t n, int K, SubmGeom g, const uint2* __restrict__ wr, int64_t nw,
+    const uint2* __restrict__ col_e, const int32_t* __restrict__ n_unique,
+    const int32_t* __restrict__ n_extra, int32_t* __restrict__ cols_row, int32_t* __restrict__ nbr,
+    int32_t* __restrict__ blk_cnt, int nblk, uint32_t* __restrict__ col_masks,
+    const uint8_t* __restrict__ touched) {
+  constexpr int KX = 5, R = 5;  // R kernel rows have their loads in flight together
+  __shared__ int32_t s_cnt[kRows / kWave][kProbe5Slots];
+  const int t = threadIdx.x;
+  const int lane = t & (kWave - 1);
+  const uint32_t un = static_cast<uint32_t>(n);  // 0 < n < 2^29
+  const uint32_t col_t = blockIdx.x * static_cast<uint32_t>(kRows) + static_cast<uint32_t>(t);
+  // lanes past the last column work as the last column and store the same
+  // values to it; the counts leave them out
+  const uint64_t real = __ballot(col_t < un);
+  const uint32_t col = col_t < un ? col_t : un - 1;
+  const bool live = col < static_cast<uint32_t>(*n_unique + *n_extra);  // the other columns are empty
+  const uint2 me = live ? col_e[col] : make_uint2(0u, 0u);
+  cols_row[col] = static_cast<int32_t>(me.x) - 1;
+  const int4 c = cell_coords(g, me.y);  // (b, z, y, x)
+  const int x_lo = c.w - KX / 2;
+  const int x_first = x_lo > 0 ? x_lo : 0;  // the row's first cell inside the grid
+  const uint32_t shift = static_cast<uint32_t>(x_first - x_lo);
+  const uint32_t W = static_cast<uint32_t>(g.shape.x);
+  uint32_t vmask = 0;
+#pragma unroll
+  for (int kx = 0; kx < KX; ++kx) vmask |= (static_cast<uint32_t>(x_lo + kx) < W ? 1u : 0u) << kx;
+  const uint32_t key_first = me.y + static_cast<uint32_t>(x_first - c.w);
+  const uint32_t D = static_cast<uint32_t>(g.shape.z), H = static_cast<uint32_t>(g.shape.y);
+  const uint32_t last_w = static_cast<uint32_t>(nw - 1);
+  const char* const ce = reinterpret_cast<const char*>(col_e);
+  const uint32_t col4 = col << 2;
+  const uint64_t slot_bytes = static_cast<uint64_t>(n) * sizeof(int32_t);
+  global_char* slot = (global_char*)nbr;
+  const int n_rows = g.ks.z * g.ks.y;
+  uint32_t cmask = 0;
+  int kz = 0, ky = 0;
+  for (int q0 = 0; q0 < n_rows; q0 += R) {
+    uint2 e0[R], e1[R];
+    uint32_t lo[R], okm[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {  // rows past the last repeat it and are not stored
+      const int dz = (kz - g.ks.z / 2) * g.dil.z, dy = (ky - g.ks.y / 2) * g.dil.y;
+      const bool ok = live && static_cast<uint32_t>(c.y + dz) < D &&
+                      static_cast<uint32_t>(c.z + dy) < H && static_cast<uint32_t>(x_first) < W;
+      okm[i] = ok ? 0xffffffffu : 0u;
+      const uint32_t off = (static_cast<uint32_t>(dz) * H + static_cast<uint32_t>(dy)) * W;
+      const uint32_t base = ok ? key_first + off : 0u;
+      const uint32_t w0 = base >> 5;
+      lo[i] = base & 31u;
+      e0[i] = entry_at(wr, TOUCHED ? touched : nullptr, w0);
+      e1[i] = entry_at(wr, TOUCHED ? touched : nullptr, w0 + 1 < last_w ? w0 + 1 : last_w);
+      if (q0 + i + 1 < n_rows && ++ky == g.ks.y) {
+        ky = 0;
+        ++kz;
+      }
+    }
+    int32_t v[R][KX];
+    uint32_t h[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const uint32_t bits = __builtin_amdgcn_alignbit(e1[i].x, e0[i].x, lo[i]);
+      h[i] = (bits << shift) & vmask & okm[i];
+      const uint32_t r_e0 = e0[i].y + __popc(e0[i].x & ~(0xffffffffu << lo[i]));
+      uint32_t r0 = select_lanes(__ballot((e0[i].x >> lo[i]) != 0u), r_e0, e1[i].y);
+      r0 = h[i] ? r0 : 0u;
+#pragma unroll
+      for (int kx = 0; kx < KX; ++kx) v[i][kx] = 0;
+      if (__ballot(h[i] != 0u)) {
+        // at most one past the last unique column: inside the array's padding
+#pragma unroll
+        for (int kx = 0; kx < KX; ++kx)
+          v[i][kx] = *reinterpret_cast<const int32_t*>(
+              ce + ((r0 + __popc(h[i] & ((1u << kx) - 1u))) << 3));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int q = q0 + i;
+      if (q >= n_rows) break;
+      int32_t counts = 0;  // lane kx: the wave's hits through slot 5q + kx
+      for_each_index(
+          [&](auto kc) {
+            constexpr int kx = decltype(kc)::value;
+            const bool hit = (h[i] >> kx) & 1u;
+            write_lane<kx>(counts, static_cast<int32_t>(__popcll(__ballot(hit) & real)));
+            *(global_int*)(slot + col4) = hit ? v[i][kx] - 1 : -1;
+            slot += slot_bytes;
+            asm("" : "+s"(slot));
+          },
+          std::make_integer_sequence<int, KX>{});
+      if (lane < KX) s_cnt[t / kWave][q * KX + lane] = counts;
+      if (q * KX < 32) cmask |= h[i] << (q * KX);
+    }
+  }
+  if (col_masks) col_masks[col] = cmask;  // K <= 32
+  __syncthreads();
+  if (t < K) {
+    int32_t sum = 0;
+#pragma unroll
+    for (int w = 0; w < kRows / kWave; ++w) sum += s_cnt[w][t];
+    blk_cnt[(int64_t)t * nblk + blockIdx.x] = sum;
+  }
+}
+
 // Row-order hit counts per (slot, block) of a row-major map, for the
 // compaction offsets of the pair lists.
 __global__ void __launch_bounds__(kRows) map_count_kernel(const int32_t* __restrict__ nbr, int64_t n,
@@ -1258,8 +1376,9 @@ int tsc::subm_pairs_ws(const int32_t* coords, int64_t n, int32_t batch_size,
     subm_rank_kernel<<<ceil_div(n, 256), 256, 0, s>>>(c4, n, g, w.wr, w.n_unique, w.col,
                                                       w.n_extra, mwords, mark_gen, counts, K);
     TSC_LAUNCH_CHECK("subm_rank");
+    const bool wide5 = ks.x == 5 && dil.x == 1 && K <= kProbe5Slots && n < kProbe333Rows;
     // slots from 64 on are added into the per-block table, which starts at 0
-    if (K > 64 &&
+    if (K > 64 && !wide5 &&
         (rc = fill_u32(reinterpret_cast<uint32_t*>(blk_cnt), (int64_t)nblk * K, 0u, s)))
       return rc;
     if (ks.x == 3 && ks.y == 3 && ks.z == 3 && dil.x == 1 && n < kProbe333Rows) {
@@ -1282,6 +1401,16 @@ int tsc::subm_pairs_ws(const int32_t* coords, int64_t n, int32_t batch_size,
           n, K, g, w.wr, nw, w.col, nullptr, w.n_unique, w.n_extra, cols_row, nbr, blk_cnt,
           nblk, counts, col_masks, w.touched);
       TSC_LAUNCH_CHECK("subm_probe_rows");
+    } else if (wide5) {
+      if (w.touched)
+        subm_probe_5wide_kernel<true><<<ceil_div(n, kRows), kRows, 0, s>>>(
+            n, K, g, w.wr, nw, w.col, w.n_unique, w.n_extra, cols_row, nbr, blk_cnt, nblk,
+            col_masks, w.touched);
+      else
+        subm_probe_5wide_kernel<false><<<ceil_div(n, kRows), kRows, 0, s>>>(
+            n, K, g, w.wr, nw, w.col, w.n_unique, w.n_extra, cols_row, nbr, blk_cnt, nblk,
+            col_masks, nullptr);
+      TSC_LAUNCH_CHECK("subm_probe_5wide");
     } else {
       subm_probe_cols_kernel<<<ceil_div(n, 256), 256, 0, s>>>(n, K, g, w.wr, w.col, w.n_unique,
                                                               w.n_extra, cols_row, nbr, blk_cnt,
