@@ -41,3 +41,23 @@ def test_ragged_widths(c_in, c_out, k, dtype):
             z = _conv_raw(odd, m._packed_weight(dtype), m.bias, nbr, None, 0, n, 0)
             assert torch.equal(z[1::2], y.features[1::2])
             assert not torch.isfinite(z[::2]).any()
+
+
+@pytest.mark.parametrize("c_in,c_out", [(12, 48), (5, 40), (7, 64), (20, 96)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_column_tiles_per_wave(c_in, c_out, dtype):
+    """Row counts around the lines between one, two, three and four column
+    tiles per wave: the tiles of a wave share its gathers and nothing else, so
+    a row's bits do not depend on how many there are (the first 2900 rows of
+    each layer against a 2900-row layer, which has one, on the same map)."""
+    shape = (40, 44, 48)
+    for n in (12_736, 12_864, 25_536, 25_664, 38_336, 38_464):
+        idx = _tiny(9, shape, 1, n)
+        feats = np.random.default_rng(n).standard_normal((n, c_in)).astype(np.float32)
+        m = _module("subm", c_in, c_out, 3, dtype=dtype, seed=c_in)
+        y = _check_layer(m, feats, idx, shape, 1, dtype, rows=2000, what=f"tiles {c_out} n={n}")
+        nbr = generate_subm_indice_pairs(torch.from_numpy(idx).to(DEV), shape, 1, 3).neighbour_map(n, DEV)
+        few = nbr[:, :2900].contiguous()
+        f = torch.from_numpy(feats).to(DEV).to(dtype)
+        z = _conv_raw(f, m._packed_weight(dtype), m.bias, few, None, 0, 2900, 0)
+        assert torch.equal(z, y.features[:2900])

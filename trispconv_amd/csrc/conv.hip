@@ -2049,12 +2049,19 @@ int dispatch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, con
                     const int32_t* nbr, const int32_t* order, int nbr_ordered, int64_t n_out,
                     int K, int c_out, void* out, hipStream_t s) {
   constexpr int elem = static_cast<int>(sizeof(T));
-  // Column tiles per wave: up to 4, fewer while that leaves under 2048
-  // workgroups (each extra column group re-gathers its rows, from cache).
+  // Column tiles per wave: up to 4, fewer while that leaves the chip short of
+  // workgroups, since each extra column group gathers its rows again (from
+  // cache).  Measured per launch, f16, 1 / 2 / 4 tiles: 20->64, 15k rows (235
+  // row groups) 15.1 / 10.9 / 11.4 us, 40k rows 30.8 / 21.2 / 18.6; 3->32 with
+  // 125 slots, 80k rows 41.6 / 28.5, 3k rows 9.4 / 10.2; f32 128->20, 15k rows
+  // 69.7 / 75.1, 40k rows 168 / 145.  One and three tiles: 48->48, 40k rows
+  // 36.4 / 27.1, 150k rows 112 / 79.
   const int nt_all = static_cast<int>(ceil_div(c_out, 16));
   const int64_t blocks = ceil_div(n_out, 4 * kNarrowRows);
-  int nt = nt_all % 4 == 0 ? 4 : (nt_all % 2 == 0 ? 2 : 1);
-  while (nt > 1 && blocks * (nt_all / nt) < 2048) nt /= 2;
+  auto enough = [&](int nt, int64_t groups) {
+    return nt_all % nt == 0 && blocks * (nt_all / nt) >= groups;
+  };
+  int nt = enough(4, 600) ? 4 : enough(3, 400) ? 3 : enough(2, elem == 4 ? 400 : 200) ? 2 : 1;
   const int whole = (c_in % 8 == 0 || elem == 4) ? 16 : 8;  // bytes of an aligned piece
   const uintptr_t f = reinterpret_cast<uintptr_t>(feat);
   TSC_REQUIRE(f % elem == 0, "conv: features must be aligned to their elements");
@@ -2071,7 +2078,8 @@ int dispatch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, con
   const int piece = read == kWhole ? whole : read == kRagged ? ragged : elem;
   if (read == kSingle) nt = 1;
 #define TSC_NARROW_CASE(R_, P_, NT_)                                                            if (read == R_ && piece == P_ && nt == NT_)                                                     return launch_narrow<T, R_, P_, NT_>(feat, n_in, c_in, W, ep, nbr, order, nbr_ordered,                                             n_out, K, c_out, out, s);
-#define TSC_NARROW_CASES(R_, P_)   TSC_NARROW_CASE(R_, P_, 1) TSC_NARROW_CASE(R_, P_, 2) TSC_NARROW_CASE(R_, P_, 4)
+#define TSC_NARROW_CASES(R_, P_)   TSC_NARROW_CASE(R_, P_, 1) TSC_NARROW_CASE(R_, P_, 2) TSC_NARROW_CASE(R_, P_, 3) \
+  TSC_NARROW_CASE(R_, P_, 4)
   TSC_NARROW_CASES(kWhole, 16)
   if constexpr (sizeof(T) == 2) {
     TSC_NARROW_CASES(kWhole, 8)
