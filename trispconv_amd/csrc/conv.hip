@@ -1933,6 +1933,8 @@ int dma_per_cu(int dtype, int bn, int rb) {
 //     one tile per CU for f16/bf16 layers the direct-to-LDS kernel takes
 //     (64->64, 8k rows 14.1 against 15.7; 10k rows 18.5 against 15.9), two for
 //     a single column tile (inverse 64->32, 30k rows 15.2 against 17.1), for
+//     strided and inverse layers, whose rows use few slots (inverse 128->64,
+//     15k rows 21.4 against 27.8; strided 64->128, 6k rows 15.5 against 16.6), for
 //     K < 12 (32->64 with 8 slots, 20k rows 10.2 against 8.6) and for f32
 //     (64->64, 16k rows 48 against 50; 128->128, 16k rows 173 against 115), and
 //     two and a half for the other f16/bf16 layers (32->32, 28k rows 12.8
@@ -1967,7 +1969,7 @@ MfmaChoice choose_mfma(int dtype, int c_in, int c_out, int K, int64_t n_in, int6
     return tiles(256) < (c.bn == 128 ? 360 : f32 || K < 12 ? 300 : 128);
   };
   while (c.bn > 32 && few()) c.bn /= 2;
-  const bool two = f32 || (dma ? c_out == 32 : K < 12);
+  const bool two = f32 || (dma ? c_out == 32 || n_in != n_out : K < 12);
   const int64_t split_tiles = two ? 2 * kCus : dma ? kCus : 5 * kCus / 2;
   c.split = c.bn == 32 && K >= 8 && tiles(kSplitRows) <= split_tiles;
   c.dma = dma && !c.split;
