@@ -262,6 +262,26 @@ TSC_API int tsc_inverse_fill_ids(const int32_t* fwd_pairs_in, const int32_t* fwd
                                  const int32_t* in_ids, const int32_t* fwd_in_coords,
                                  int64_t n_fwd_in, int64_t n_out, int32_t* out_coords,
                                  int32_t* nbr, int32_t* inv_pairs_out, tsc_stream_t stream);
+/* tsc_inverse_fill_ids with the map's columns grouped by the slots they can
+ * use: an input row's residues (coordinate + padding) mod stride on the three
+ * axes decide which kernel offsets reach an output cell, so the rows of one
+ * residue class have (away from the grid's borders) one slot set.  Column t of
+ * nbr [K][n_out] belongs to output row cols_row[t]; classes with more slots
+ * come first, rows ascend within a class.  out_coords, cols_row's rows and
+ * inv_pairs_out are as in tsc_inverse_fill_ids.  Needs at most 64 classes (the
+ * product of the strides). */
+TSC_API int64_t tsc_inverse_grouped_workspace_bytes(int64_t n_fwd_in,
+                                                    const int32_t stride[3] /* host */);
+TSC_API int tsc_inverse_fill_grouped(const int32_t* fwd_pairs_in, const int32_t* fwd_pairs_out,
+                                     const int32_t* fwd_counts, int32_t k_vol, int64_t cap,
+                                     const int32_t* in_ids, const int32_t* fwd_in_coords,
+                                     int64_t n_fwd_in, const int32_t ksize[3] /* host */,
+                                     const int32_t stride[3] /* host */,
+                                     const int32_t padding[3] /* host */,
+                                     const int32_t dilation[3] /* host */, void* ws,
+                                     int64_t ws_bytes, int64_t n_out, int32_t* out_coords,
+                                     int32_t* cols_row, int32_t* nbr, int32_t* inv_pairs_out,
+                                     tsc_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Execution order for the convolution: output rows in spatial order, cut into
@@ -290,6 +310,10 @@ TSC_API int tsc_conv_plan(const int32_t* nbr, const int32_t* cols_row, int32_t r
                           int32_t batch_size, const int32_t out_spatial[3] /* host */,
                           int64_t region_rows, void* ws, int64_t ws_bytes, int32_t* order,
                           int32_t* nbr_ordered, int32_t* pos_masks, tsc_stream_t stream);
+/* masks[t] = the slot mask of column t of a map [K][n], K <= 32 (bit k set when
+ * nbr[k][t] >= 0): the row of masks a convolution reads with nbr_ordered = 2. */
+TSC_API int tsc_map_masks(const int32_t* nbr, int64_t n, int32_t k_vol, int32_t* masks,
+                          tsc_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Weights.  Replaces normalize_spconv_weight (trispconv/pytorch/weight.py:8-50)
@@ -368,9 +392,11 @@ TSC_API int tsc_conv_forward_tile(const void* feat, int32_t dtype, int64_t n_in,
                                   int64_t n_out, int32_t k_vol, int32_t c_out,
                                   int32_t column_tile, void* out, tsc_stream_t stream);
 
-/* Name of the kernel tsc_conv_forward launches for a layer of this shape
- * ("conv_mfma_kernel", "conv_dma_kernel", "conv_split_kernel" or
- * "conv_narrow_kernel"; "" for invalid sizes): what a kernel trace lists it under.  No counterpart in the reference; for profilers and benchmarks. */
+/* Name of the kernel tsc_conv_forward launches for a layer of this shape with
+ * as many input as output rows (others may take conv_split_kernel up to twice
+ * as many rows): "conv_mfma_kernel", "conv_dma_kernel", "conv_split_kernel" or
+ * "conv_narrow_kernel"; "" for invalid sizes.  What a kernel trace lists it
+ * under.  No counterpart in the reference; for profilers and benchmarks. */
 TSC_API const char* tsc_conv_kernel_name(int32_t dtype, int32_t c_in, int32_t c_out,
                                          int32_t k_vol, int64_t n_out);
 

@@ -635,3 +635,15 @@ extern "C" int tsc_conv_plan(const int32_t* nbr, const int32_t* cols_row, int32_
   }
   return 0;
 }
+
+extern "C" int tsc_map_masks(const int32_t* nbr, int64_t n, int32_t k_vol, int32_t* masks,
+                             tsc_stream_t stream) {
+  TSC_REQUIRE(n >= 0 && n < (int64_t(1) << 31) && k_vol > 0 && k_vol <= 32,
+              "map_masks: invalid sizes");
+  if (n == 0) return 0;
+  TSC_REQUIRE(nbr && masks, "map_masks: null pointer");
+  row_mask_kernel<<<ceil_div(n, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+      nbr, n, k_vol, reinterpret_cast<uint32_t*>(masks), nullptr);
+  TSC_LAUNCH_CHECK("map_masks");
+  return 0;
+}

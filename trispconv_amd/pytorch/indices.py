@@ -123,6 +123,8 @@ class IndiceData:
         self._map_cols: Optional[torch.Tensor] = None
         self._cols_row: Optional[torch.Tensor] = None
         self._raster = False
+        # an inverse whose columns are grouped by the slots they can use
+        self._grouped = False
         # the output rows themselves are in (b,z,y,x) order (strided builds
         # emit the sorted unique output set)
         self._rows_raster = False
@@ -142,6 +144,8 @@ class IndiceData:
         # strided builds: each input row's id among the rows with a pair (-1
         # for the others), the inverse's output ids
         self._in_ids: Optional[torch.Tensor] = None
+        # and their geometry as ABI arguments
+        self._geo: Optional[tuple] = None
         # input rows the pairs may name: ids lie in [0, _in_bound) (the
         # builders' input rows; for user-assigned lists their largest id + 1)
         self._in_bound: Optional[int] = None
@@ -261,7 +265,7 @@ class IndiceData:
     def _drop_tables(self) -> None:
         self._pin = self._pout = self._cnt = self._nbr = self._order = None
         self._map_cols = self._cols_row = None
-        self._raster = False
+        self._raster = self._grouped = False
         self._map_masks = False
         self._nbr_ordered = None
         self._inverse_cache = None
@@ -275,7 +279,7 @@ class IndiceData:
         ``n_in``: the rows of the features the map will gather from (checked
         against user-assigned lists)."""
         if self._nbr is None and self._map_cols is not None:
-            if not self._raster:  # the builder's columns are the rows in order
+            if not (self._raster or self._grouped):  # the builder's columns are the rows in order
                 self._nbr = self._map_cols
             else:
                 nbr = torch.full((self.K, n_out), -1, dtype=torch.int32, device=device)
@@ -419,6 +423,16 @@ class IndiceData:
                 or self._slot_repeat != 1:
             return None
         region = int(min(max(_REGION_BYTES // max(int(row_bytes), 1), 2048), 1 << 30))
+        if self._grouped and n_out <= region:
+            # the columns already are what a sort by slot mask would give;
+            # a second use adds their masks, which shorten its set-up
+            self._conv_uses += 1
+            if self._conv_uses == 2 and self.K <= 32:
+                base = self._map_cols.data_ptr()
+                L.check(L.lib().tsc_map_masks(base, n_out, self.K, base + 4 * self.K * n_out,
+                                              L.stream_of(self._map_cols)), "map masks")
+                self._map_masks = True
+            return None
         if self._order is None or self._order_region != region:
             self._conv_uses += 1
             raster = self._raster if self._map_cols is not None else self._rows_raster
@@ -486,7 +500,7 @@ class IndiceData:
         order = self.execution_order(n_out, device, row_bytes)
         if order is not None:
             return self._nbr_ordered, order, self._ordered_flag
-        if self._map_cols is not None and self._raster:
+        if self._map_cols is not None and (self._raster or self._grouped):
             return self._map_cols, self._cols_row, 2 if self._map_masks else 1
         return self.neighbour_map(n_out, device), None, 0
 
@@ -827,6 +841,7 @@ def generate_strided_indice_pairs(indices: torch.Tensor, spatial_shape, batch_si
         batch_size=int(batch_size), rows_raster=True)
     data._n_in_paired = int(host[K + 2])
     data._in_ids = tables[o_ids:o_ids + n]
+    data._geo = sz.geo
     _STRIDED_BITMAPS[out_coords] = (ws, sz.out_words, tuple(out_shape), int(batch_size),
                                     out_coords._version,
                                     (out_coords.data_ptr(), out_coords.storage_offset()))
@@ -869,6 +884,70 @@ def _strided_sizes(n, batch_size, shape, ks, st, pd, dil, out_shape) -> _Strided
     return _StridedSizes(n, batch_size, shape, ks, st, pd, dil, out_shape)
 
 
+# A convolution over an inverse map in row order runs nearly every slot for
+# every tile; over grouped columns, only those its rows have.  Grouping takes
+# two more launches, so it is done where the former is some 40 us or more of
+# matrix work: multiply-adds over all slots times 2, f32 ones counted three
+# times (the rate such layers reach: 250 TFLOP/s f16, 85 f32).  Measured, down
+# and up again on new voxels: 128->64 f32, 8.5k rows 231 -> 186 us; 64->32
+# bf16, 250k rows (27e9) 196 -> 177; 60k rows (6.6e9), where the host's time
+# hides the convolution, 128 -> 152.
+_GROUP_MIN_WORK = 10_000_000_000
+
+
+def _group_inverse(fwd: IndiceData, n_out: int, channel_work: int) -> bool:
+    """Whether the inverse of ``fwd`` gets its columns grouped by the slots they
+    can use: strides that leave more than one residue class, and a layer that
+    skips unused slots (``channel_work`` > 0, see inverse_pairs_for)."""
+    st = fwd.stride
+    return fwd._geo is not None and 1 < st[0] * st[1] * st[2] <= 64 \
+        and 2 * n_out * fwd.K * channel_work >= _GROUP_MIN_WORK
+
+
+@functools.lru_cache(maxsize=64)
+def _grouped_ws_bytes(n_in: int, stride) -> int:
+    return int(L.lib().tsc_inverse_grouped_workspace_bytes(n_in, L.i3(stride)))
+
+
+def _grouped_inverse(fwd: IndiceData, in_coords: torch.Tensor, n_out: int, stream) -> IndiceData:
+    """The inverse of a strided build made here, its map by grouped columns."""
+    lib, dev, K, n_in = L.lib(), fwd._pin.device, fwd.K, len(fwd.input_indices)
+    cap = fwd._pin.shape[1]
+    _, ks, st, pd, dil, _ = fwd._geo
+    ws_bytes = _grouped_ws_bytes(n_in, fwd.stride)
+    ws = L.workspace(ws_bytes, dev)
+    out_coords = torch.empty((n_out, 4), dtype=torch.int32, device=dev)
+    # cols_row, the map with room for its slot masks as row K, the pair table
+    o_map = _align64(n_out)
+    o_pout = o_map + _align64((K + 1) * n_out)
+    tables = torch.empty(o_pout + K * cap, dtype=torch.int32, device=dev)
+    base = tables.data_ptr()
+    L.check(lib.tsc_inverse_fill_grouped(
+        fwd._pin.data_ptr(), fwd._pout.data_ptr(), fwd._cnt.data_ptr(), K, cap,
+        fwd._in_ids.data_ptr(), in_coords.data_ptr(), n_in, ks, st, pd, dil, ws.data_ptr(),
+        ws_bytes, n_out, out_coords.data_ptr(), base, base + 4 * o_map, base + 4 * o_pout, stream),
+        "inverse pairs")
+    d = IndiceData._from_tables(
+        out_indices=out_coords, input_indices=fwd.out_indices,
+        input_spatial_shape=fwd.output_spatial_shape,
+        output_spatial_shape=fwd.input_spatial_shape, kernel_size=fwd.kernel_size,
+        stride=fwd.stride, padding=fwd.padding, dilation=fwd.dilation, subm=False,
+        pin=fwd._pout, pout=tables[o_pout:].view(K, cap), cnt_dev=fwd._cnt, pair_num=fwd.pair_num,
+        nbr=None, batch_size=fwd._batch_size, map_cols=tables[o_map:o_map + K * n_out].view(K, n_out),
+        cols_row=tables[:n_out])
+    d._grouped = True
+    return d
+
+
+def inverse_pairs_for(fwd: IndiceData, c_in: int, c_out: int, dtype: torch.dtype) -> IndiceData:
+    """generate_inverse_indice_pairs for a layer of c_in -> c_out channels
+    computed in ``dtype``: the same pairs, their map laid out for it."""
+    # the 32x32-tile kernels skip unused slots, the narrow one runs them all
+    tiled = c_in % 16 == 0 and c_out % 32 == 0 and fwd.K <= 64
+    work = c_in * c_out * (3 if dtype == torch.float32 else 1) if tiled else 0
+    return _inverse_pairs(fwd, work)
+
+
 def generate_inverse_indice_pairs(fwd: IndiceData) -> IndiceData:
     """Pairs of the inverse of a strided layer (modules.py:175-212).
 
@@ -876,6 +955,10 @@ def generate_inverse_indice_pairs(fwd: IndiceData) -> IndiceData:
     slot k reads forward outputs pairs_out[k] and writes the compact id of
     forward input pairs_in[k]; pair_num is the forward's.
     """
+    return _inverse_pairs(fwd, 0)
+
+
+def _inverse_pairs(fwd: IndiceData, channel_work: int) -> IndiceData:
     fwd._ensure_tables()
     from_lists = fwd._pin is None
     if from_lists:
@@ -897,6 +980,8 @@ def generate_inverse_indice_pairs(fwd: IndiceData) -> IndiceData:
         # a forward built here: its fill gave every input row its output id
         # and its count read gave the row count, so the inverse is one fill
         n_out = fwd._n_in_paired
+        if _group_inverse(fwd, n_out, channel_work):
+            return _grouped_inverse(fwd, in_coords, n_out, stream)
         out_coords = torch.empty((n_out, 4), dtype=torch.int32, device=dev)
         nbr = torch.empty((K, n_out), dtype=torch.int32, device=dev)
         inv_pout = torch.empty((K, cap), dtype=torch.int32, device=dev)

@@ -17,8 +17,8 @@ import torch
 import torch.nn as nn
 
 from .functional import Epilogue, compute_dtype, dense_forward, sparse_conv_forward
-from .indices import (IndiceData, _output_spatial_shape, _to3, generate_inverse_indice_pairs,
-                      generate_strided_indice_pairs, generate_subm_indice_pairs)
+from .indices import (IndiceData, _output_spatial_shape, _to3, generate_strided_indice_pairs,
+                      generate_subm_indice_pairs, inverse_pairs_for)
 from .tensor import SparseConvTensor
 from .weight import ConvWeight, PackedWeight, normalize_spconv_weight, pack_weight, weight_state
 
@@ -180,7 +180,7 @@ class SparseConvolution(SparseModule):
             return _derived(x, out, x.indices, x.spatial_shape)
         inv = fwd._inverse_cache
         if inv is None:
-            inv = generate_inverse_indice_pairs(fwd)
+            inv = inverse_pairs_for(fwd, self.in_channels, self.out_channels, packed.dtype)
             fwd._inverse_cache = inv
         n_out = len(inv.out_indices)
         out = sparse_conv_forward(x.features, packed, self.bias, inv, n_out, epilogue)
