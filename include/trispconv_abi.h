@@ -233,6 +233,21 @@ TSC_API int tsc_strided_fill(const int32_t* coords, int64_t n, int32_t batch_siz
                      const int32_t* counts, int64_t out_cap, int32_t* out_coords, int32_t* nbr,
                      int32_t* pairs_in, int32_t* pairs_out, int32_t* in_ids,
                      tsc_stream_t stream);
+/* Both phases in one call, which returns with the K + 3 counts in counts_host
+ * while the fill may still run on the stream; the same buffers and rules (when
+ * counts_host[K] > out_cap, call tsc_strided_fill with room for that many rows).
+ * Not for graph capture: it waits for the counts. */
+TSC_API int tsc_strided_build(const int32_t* coords, int64_t n, int32_t batch_size,
+                              const int32_t spatial[3] /* host */,
+                              const int32_t ksize[3] /* host */,
+                              const int32_t stride[3] /* host */,
+                              const int32_t padding[3] /* host */,
+                              const int32_t dilation[3] /* host */,
+                              const int32_t out_spatial[3] /* host */, void* ws, int64_t ws_bytes,
+                              void* marks, int64_t marks_size, int32_t gen, int32_t* counts,
+                              int32_t* counts_host /* host */, int64_t out_cap,
+                              int32_t* out_coords, int32_t* nbr, int32_t* pairs_in,
+                              int32_t* pairs_out, int32_t* in_ids, tsc_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Inverse pairs.  Replaces the pair swap of SparseInverseConv3d

@@ -8,8 +8,8 @@ device as padded int32 tables (slot k owns ``[k, :pair_num[k]]``) next to the
 output-major neighbour map the convolution reads; the reference-style lists
 of K int64 tensors are materialised on first access to ``pairs_in`` /
 ``pairs_out``.  ``pair_num`` is a CPU int64 tensor, as in the reference
-(indices.py:131): strided builds read it with the one device-to-host copy
-they make (their output count), submanifold builds on its first access.
+(indices.py:131): strided builds read it with their output count, submanifold
+builds on its first access.
 """
 from __future__ import annotations
 
@@ -111,6 +111,9 @@ class IndiceData:
         # reading them on the build's stream, or None);
         # counts[K] holds the build's status flags
         self._counts_pending: Optional[Tuple[torch.Tensor, int, Optional[Callable[[], None]]]] = None
+        # a strided build's counts on the host ([K + 3], a ctypes array), from
+        # which pair_num is made when it is read
+        self._host_counts = None
         self._pairs_in = pairs_in
         self._pairs_out = pairs_out
         # device tables
@@ -176,11 +179,13 @@ class IndiceData:
                                    "the strided build they were registered with")
             self._pair_num = host[:K].long()
             self._counts_pending = None
+        elif self._pair_num is None and self._host_counts is not None:
+            self._pair_num = torch.tensor(self._host_counts[:self.K], dtype=torch.int64)
         return self._pair_num
 
     def _set_pair_num(self, value: torch.Tensor) -> None:
         self._pair_num = value
-        self._counts_pending = None
+        self._counts_pending = self._host_counts = None
 
     # --------------------------------------------------- construction
     @classmethod
@@ -788,21 +793,15 @@ def generate_strided_indice_pairs(indices: torch.Tensor, spatial_shape, batch_si
     counts = torch.empty(K + 3, dtype=torch.int32, device=dev)
     stream = L.stream_of(coords)
     marks, marks_size, gen = _marks_for(dev, stream, sz.marks_bytes)
-    L.check(lib.tsc_strided_count(coords.data_ptr(), n, int(batch_size), *sz.geo, ws.data_ptr(),
-                                  sz.ws_bytes, marks, marks_size, gen, counts.data_ptr(), stream),
-            "generate_strided_indice_pairs")
-    # the counts go to the host behind the count pass; the fill is queued
-    # before they arrive, with room for the rows this geometry's largest
-    # output ratio so far predicts, and is queued again at the exact size in
-    # the rare build that outgrows it
-    host = torch.empty(K + 3, dtype=torch.int32, pin_memory=True)
-    host.copy_(counts, non_blocking=True)
-    counted = torch.cuda.Event()
-    counted.record(torch.cuda.current_stream(dev))
+    # one call counts, queues the fill before the counts reach the host, with
+    # room for the rows this geometry's largest output ratio so far predicts,
+    # and returns with the counts; the fill is queued again at the exact size
+    # in the rare build that outgrows that room
+    host = sz.host_counts()
     geo_key = (int(batch_size), shape, ks, st, pd, dil)
     cap = _strided_out_cap(geo_key, n, sz.cells)
 
-    def fill(out_cap: int):
+    def outputs(out_cap: int):
         # the output coordinates (the next tensor's indices, with their own
         # storage and version counter); the map and the two pair tables in
         # one allocation at 256-byte aligned offsets, passed as raw
@@ -812,22 +811,23 @@ def generate_strided_indice_pairs(indices: torch.Tensor, spatial_shape, batch_si
         tables = torch.empty(max(o_pin + 2 * _align64(K * n) + n, 1), dtype=torch.int32,
                              device=dev)
         base = tables.data_ptr()
-        L.check(lib.tsc_strided_fill(coords.data_ptr(), n, int(batch_size), *sz.geo,
-                                     ws.data_ptr(), sz.ws_bytes, counts.data_ptr(), out_cap,
-                                     out_coords.data_ptr(), base, base + 4 * o_pin,
-                                     base + 4 * (o_pin + _align64(K * n)),
-                                     base + 4 * (o_pin + 2 * _align64(K * n)), stream),
-                "generate_strided_indice_pairs")
-        return out_coords, tables, o_pin
+        return out_coords, tables, o_pin, (out_cap, out_coords.data_ptr(), base, base + 4 * o_pin,
+                                           base + 4 * (o_pin + _align64(K * n)),
+                                           base + 4 * (o_pin + 2 * _align64(K * n)), stream)
 
-    out_coords, tables, o_pin = fill(cap)
-    counted.synchronize()
+    out_coords, tables, o_pin, args = outputs(cap)
+    L.check(lib.tsc_strided_build(coords.data_ptr(), n, int(batch_size), *sz.geo, ws.data_ptr(),
+                                  sz.ws_bytes, marks, marks_size, gen, counts.data_ptr(), host,
+                                  *args), "generate_strided_indice_pairs")
     _raise_status(int(host[K + 1]), "generate_strided_indice_pairs")
-    n_out = int(host[K])
+    n_out = host[K]
     if n > 0:
         _STRIDED_OUT_RATIO[geo_key] = max(_STRIDED_OUT_RATIO.get(geo_key, 0.0), n_out / n)
     if n_out > cap:
-        out_coords, tables, o_pin = fill(n_out)
+        out_coords, tables, o_pin, args = outputs(n_out)
+        L.check(lib.tsc_strided_fill(coords.data_ptr(), n, int(batch_size), *sz.geo,
+                                     ws.data_ptr(), sz.ws_bytes, counts.data_ptr(), *args),
+                "generate_strided_indice_pairs")
     out_coords = out_coords[:n_out]
     o_pout = o_pin + _align64(K * n)
     o_ids = o_pout + _align64(K * n)
@@ -837,9 +837,10 @@ def generate_strided_indice_pairs(indices: torch.Tensor, spatial_shape, batch_si
     data = IndiceData._from_tables(
         out_indices=out_coords, input_indices=indices, input_spatial_shape=shape,
         output_spatial_shape=out_shape, kernel_size=ks, stride=st, padding=pd, dilation=dil,
-        subm=False, pin=pin, pout=pout, cnt_dev=counts[:K], pair_num=host[:K].long(), nbr=nbr,
+        subm=False, pin=pin, pout=pout, cnt_dev=counts[:K], pair_num=None, nbr=nbr,
         batch_size=int(batch_size), rows_raster=True)
-    data._n_in_paired = int(host[K + 2])
+    data._host_counts = host
+    data._n_in_paired = host[K + 2]
     data._in_ids = tables[o_ids:o_ids + n]
     data._geo = sz.geo
     _STRIDED_BITMAPS[out_coords] = (ws, sz.out_words, tuple(out_shape), int(batch_size),
@@ -860,6 +861,7 @@ class _StridedSizes:
             n, K, batch_size, self.geo[5], int(self.marks_bytes > 0))), 1)
         self.cells = batch_size * out_shape[0] * out_shape[1] * out_shape[2]
         self.out_words = (self.cells + 31) // 32
+        self.host_counts = ctypes.c_int32 * (K + 3)
 
 
 # Largest n_out / n each strided geometry (batch size, input shape, kernel,
