@@ -24,9 +24,11 @@ def _exact(feats, m, nbr):
     return out
 
 
-# rows: one partial tile of the register-gather kernel (C_in = 48), the
-# direct-to-LDS kernel at 32 and at 64 rows per wave
-@pytest.mark.parametrize("c_in,c_out,n,grid,tile", [(48, 64, 9000, 40, 0), (64, 64, 150_001, 96, 0),
+# the slot-split kernel (rows of one partial tile and of several), the
+# register-gather kernel (C_in = 48), the direct-to-LDS kernel at 32 and at 64
+# rows per wave
+@pytest.mark.parametrize("c_in,c_out,n,grid,tile", [(48, 64, 20_000, 40, 0), (64, 64, 50, 12, 0),
+                                                    (48, 32, 3000, 24, 0), (64, 64, 150_001, 96, 0),
                                                     (64, 64, 300_007, 128, 0), (32, 32, 30_000, 64, 0),
                                                     (64, 128, 5000, 32, 128)])
 @pytest.mark.parametrize("scale", [1.0, 1e-12, 1e15])
@@ -68,4 +70,8 @@ def test_split_precision_and_non_finite_rows(c_in, c_out, n, grid, tile, scale):
     assert torch.equal(a[inf], b[inf])
     own = (nbr == n - 1).any(0) & ~((nbr == 3) | (nbr == n // 2)).any(0)
     fin = own[:, None] & torch.isfinite(ref) & (ref.abs() < 1e38)
-    assert torch.allclose(got[fin], ref[fin], rtol=1e-3)
+    # such a sum cancels: C_in products of up to big * max|w| each, summed with a
+    # rounding of 2^-24 of at most their absolute sum at each of C_in steps
+    # (the other neighbours' products are far below)
+    bound = c_in * c_in * 2.0 ** -24 * 3.4028235e38 * float(m.weight.abs().max())
+    assert float((got[fin].double() - ref[fin].double()).abs().max()) <= bound

@@ -1429,9 +1429,23 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
       ring[S][1][u] = p1[u];
     }
   };
-  auto compute = [&](auto slot, int k) {
+  auto compute = [&](auto slot, int k, auto split) {
     constexpr int S = decltype(slot)::value;
     if (k >= K) return;
+    if constexpr (decltype(split)::value) {
+#pragma unroll
+      for (int t2 = 0; t2 < UB / 2; ++t2) {
+        const Split8 a0 = split8(ring[S][0][2 * t2], ring[S][0][2 * t2 + 1]);
+        const Split8 a1 = split8(ring[S][1][2 * t2], ring[S][1][2 * t2 + 1]);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const Split8 b = split8(bring[S][nb][2 * t2], bring[S][nb][2 * t2 + 1]);
+          acc[0][nb] = mfma_split(a0, b, acc[0][nb]);
+          acc[1][nb] = mfma_split(a1, b, acc[1][nb]);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < UB; ++u) {
 #pragma unroll
@@ -1458,66 +1472,90 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
     }
   };
 
-  int kc = -1, cc = nch - 1;
-  advance(kc, cc);  // this wave's first slot
-  int kn = kc, cn = cc;
-  advance(kn, cn);
-  load_b(Slot<0>{}, kc, cc);
-  load_a(Slot<0>{}, kc, cc);
-  auto body = [&](auto slot) {
-    constexpr int S = decltype(slot)::value;
-    load_b(Slot<(S + 1) % 2>{}, kn, cn);  // next stage's weights
-    load_a(Slot<(S + 1) % 2>{}, kn, cn);  // and operands
-    __builtin_amdgcn_sched_barrier(0);
-    compute(Slot<S>{}, kc);
-    kc = kn;
-    cc = cn;
+  auto run = [&](auto split) {
+    int kc = -1, cc = nch - 1;
+    advance(kc, cc);  // this wave's first slot
+    int kn = kc, cn = cc;
     advance(kn, cn);
-  };
-  while (kc < K) {
-    body(Slot<0>{});
-    body(Slot<1>{});
-  }
-
-  // ---- waves 1-3 hand their partial sums to wave 0, which adds them in wave
-  // order and stores.  32x32 accumulator layout: register i of lane l holds
-  // row (i/4)*8 + (l/32)*4 + i%4 and column l%32 of the block.
-  if (wave > 0) {
-    float* dst = s_part + (wave - 1) * PART;
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dst[((rb * NB + nb) * 16 + i) * 64 + lane] = acc[rb][nb][i];
-  }
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int w = 0; w < 3; ++w)
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          acc[rb][nb][i] += s_part[w * PART + ((rb * NB + nb) * 16 + i) * 64 + lane];
-  const bool affine = ep.mean != nullptr;
-  const bool relu = ep.relu != 0;
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = rb * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-      const int32_t orow = s_orow[row];
-      if (orow < 0) continue;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const int cl = nb * 32 + (lane & 31);
-        out[(int64_t)orow * c_out + nbt * BN + cl] =
-            from_f32<T>(finish(acc[rb][nb][i] + s_bias[cl], s_scale[cl], s_shift[cl], affine, relu));
-      }
+    load_b(Slot<0>{}, kc, cc);
+    load_a(Slot<0>{}, kc, cc);
+    auto body = [&](auto slot) {
+      constexpr int S = decltype(slot)::value;
+      load_b(Slot<(S + 1) % 2>{}, kn, cn);  // next stage's weights
+      load_a(Slot<(S + 1) % 2>{}, kn, cn);  // and operands
+      __builtin_amdgcn_sched_barrier(0);
+      compute(Slot<S>{}, kc, split);
+      kc = kn;
+      cc = cn;
+      advance(kn, cn);
+    };
+    while (kc < K) {
+      body(Slot<0>{});
+      body(Slot<1>{});
     }
+    // waves 1-3 hand their partial sums to wave 0, which adds them in wave order
+    if (wave > 0) {
+      float* dst = s_part + (wave - 1) * PART;
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) dst[((rb * NB + nb) * 16 + i) * 64 + lane] = acc[rb][nb][i];
+    }
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int w = 0; w < 3; ++w)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            acc[rb][nb][i] += s_part[w * PART + ((rb * NB + nb) * 16 + i) * 64 + lane];
+  };
+  // wave 0 stores the elements that `which` picks.  32x32 accumulator layout:
+  // register i of lane l holds row (i/4)*8 + (l/32)*4 + i%4 and column l%32 of
+  // the block.
+  auto store = [&](auto which) {
+    const bool affine = ep.mean != nullptr;
+    const bool relu = ep.relu != 0;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int row = rb * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+        const int32_t orow = s_orow[row];
+        if (orow < 0) continue;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const int cl = nb * 32 + (lane & 31);
+          if (which(rb, nb, i))
+            out[(int64_t)orow * c_out + nbt * BN + cl] =
+                from_f32<T>(finish(acc[rb][nb][i] + s_bias[cl], s_scale[cl], s_shift[cl], affine, relu));
+        }
+      }
+  };
+  run(std::bool_constant<F32>{});
+  auto every = [](int, int, int) { return true; };
+  if constexpr (!F32) {
+    if (wave == 0) store(every);
+  } else {
+    NonFinite<2, NB> bad;
+    if (wave == 0) {
+      store(every);
+      bad.find(acc);
+    }
+    // accumulators that are not finite once more on the f32 unit (above)
+    if (!__syncthreads_or(wave == 0 && NonFinite<2, NB>::any(acc))) return;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) acc[rb][nb] = f32x16{};
+    run(std::false_type{});
+    if (wave == 0) store([&](int rb, int nb, int i) { return bad.has(rb, nb, i); });
+  }
 }
 
 // --------------------------------------------------------- narrow MFMA --
@@ -1994,7 +2032,7 @@ int dispatch_mfma(const void* feat, int64_t n_in, int c_in, const void* W, const
       if (ch.split)                                                                          \
         return launch_split<T, BN_, CK_>(feat, c_in, W, ep, nbr, order, nbr_ordered, n_out,  \
                                          K, c_out, out, s);                                  \
-    if constexpr (CK_ * sizeof(T) == 128)                                                    \
+    if constexpr (CK_ * sizeof(T) == 128 && !(sizeof(T) == 4 && BN_ == 128))                 \
       if (ch.dma)                                                                            \
         return ch.rb == 1 ? launch_dma<T, BN_, 1>(feat, c_in, W, ep, nbr, order, nbr_ordered,  \
                                                   n_out, K, c_out, out, s)                   \
