@@ -31,7 +31,7 @@ def _exact(feats, m, nbr):
                                                     (48, 32, 3000, 24, 0), (64, 64, 150_001, 96, 0),
                                                     (64, 64, 300_007, 128, 0), (32, 32, 30_000, 64, 0),
                                                     (64, 128, 5000, 32, 128)])
-@pytest.mark.parametrize("scale", [1.0, 1e-12, 1e15])
+@pytest.mark.parametrize("scale", [1.0, 1e-12, 1e15, 1e-34])
 def test_split_precision_and_non_finite_rows(c_in, c_out, n, grid, tile, scale):
     """Against float64: at most 27 * C_in products summed in f32, so a random
     walk of that many roundings of 2^-24 bounds the relative 2-norm error

@@ -17,7 +17,7 @@
 //
 // Two code shapes share that structure:
 //   * mfma: f32/f16/bf16 with C_in a multiple of 16, C_out of 32 and K <= 64
-//     — v_mfma_f32_32x32x16_{f16,bf16} or v_mfma_f32_32x32x2_f32, 4 waves x
+//     — v_mfma_f32_32x32x16_{f16,bf16} (f32 as three bf16 values), 4 waves x
 //     (64 rows x BN cols) per tile.
 //   * narrow: every other layer (a LiDAR encoder's 4 -> 16 or 5 -> 16 first
 //     layer, 16-wide outputs, 20 class scores, K > 64) —
@@ -143,8 +143,8 @@ __device__ __forceinline__ float src_weight(const void* w, int dt, int layout, i
 // the channels c*CK + h*CK/2 + u*(16/sizeof(T)) + 0.. of chunk c: the same
 // channel split the A operand uses, so that each lane's A data is a
 // contiguous CK/2-channel (64-byte) run of a row.  An f16/bf16 MFMA step
-// (32x32x16) takes one 16-byte vector per lane; an f32 step (32x32x2) one
-// element of it.
+// (32x32x16) takes one 16-byte vector per lane, an f32 one two of them (split
+// into three bf16 operands), a step of the f32 unit (32x32x2) one element.
 template <typename T>
 __global__ void pack_mfma_kernel(const void* w, int w_dt, int layout, int K, int c_in, int c_out,
                                  int ck, T* packed) {
@@ -258,8 +258,11 @@ template <> struct MfmaOp<float> {
 // LiDAR voxels 4.4e-7 and 3.7e-7.  Their times (the first's launch, the
 // second's whole frame with its build and plan): 179 -> 133 us, 301 -> 251 us.
 // A value that is not finite or rounds to infinity in bf16 makes its products
-// NaN; the accumulators that end up not finite are computed once more on the
-// f32 unit (rerun below), so such outputs are what that unit gives.
+// NaN, and below 2^-109 lo runs out of bf16's exponents (an absolute error of
+// up to 2^-126, were such numbers flushed).  The accumulators that end up not
+// finite or below 2^-80 without being zero are computed once more on the f32
+// unit (Redo below), so such outputs are what that unit gives; in the others
+// 27 x 64 errors of 2^-126 are below 2^-35 of the sum.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
@@ -320,20 +323,27 @@ __device__ __forceinline__ Split8 load_split(const uint4* slab, int nb, int t, i
   return {plane(0), plane(1), plane(2)};
 }
 
-// The elements of this lane's accumulators that are not finite, one bit each.
+// The elements of this lane's accumulators that the f32 unit computes again:
+// not finite, or too small for the split (0 < |x| < 2^-80).  One bit each.
 template <int RB, int NB>
-struct NonFinite {
+struct Redo {
+  static constexpr uint32_t kSmall = 47u << 24;  // 2^-80's bits without the sign, shifted left
   uint32_t bits[(RB * NB + 1) / 2];
-  // whether there are any: 0 * x is 0 for every finite x, else NaN
+  // whether there are any: 0 * x is 0 for every finite x, else NaN; a zero
+  // passes the other check, as the largest value
   static __device__ __forceinline__ bool any(const f32x16 (&acc)[RB][NB]) {
     float z = 0.f;
+    uint32_t least = 0xffffffffu;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) z = fmaf(acc[rb][nb][i], 0.f, z);
-    return !(z == 0.f);
+        for (int i = 0; i < 16; ++i) {
+          z = fmaf(acc[rb][nb][i], 0.f, z);
+          least = min(least, (__float_as_uint(acc[rb][nb][i]) << 1) - 1u);
+        }
+    return !(z == 0.f) || least < kSmall - 1u;
   }
   __device__ __forceinline__ void find(const f32x16 (&acc)[RB][NB]) {
     for (uint32_t& b : bits) b = 0;
@@ -343,7 +353,8 @@ struct NonFinite {
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const bool bad = (__float_as_uint(acc[rb][nb][i]) & 0x7f800000u) == 0x7f800000u;
+          const uint32_t v = __float_as_uint(acc[rb][nb][i]) << 1;
+          const bool bad = v >= 0xff000000u || v - 1u < kSmall - 1u;
           const int e = (rb * NB + nb) * 16 + i;
           bits[e / 32] |= (bad ? 1u : 0u) << (e % 32);
         }
@@ -663,7 +674,7 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   };
   run(std::bool_constant<F32>{});
   bool rerun = false;
-  if constexpr (F32) rerun = __syncthreads_or(NonFinite<2, NB>::any(acc));
+  if constexpr (F32) rerun = __syncthreads_or(Redo<2, NB>::any(acc));
 
   // ---- epilogue: + bias (and the affine map and ReLU when asked), round
   // once, store each output element once.
@@ -728,7 +739,7 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   }
   if constexpr (F32) {
     if (rerun) {  // workgroup-uniform, and rare
-      NonFinite<2, NB> bad;
+      Redo<2, NB> bad;
       bad.find(acc);
       // the stores above are done, and the staged slot lists are read again
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1170,7 +1181,7 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   };
   run(std::bool_constant<F32>{});
   bool rerun = false;
-  if constexpr (F32) rerun = __syncthreads_or(NonFinite<RB, NB>::any(acc));
+  if constexpr (F32) rerun = __syncthreads_or(Redo<RB, NB>::any(acc));
 
   // ---- epilogue, as in conv_mfma_kernel, staged in the pool
   const bool affine = ep.mean != nullptr;
@@ -1231,7 +1242,7 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   }
   if constexpr (F32) {
     if (rerun) {  // workgroup-uniform, and rare
-      NonFinite<RB, NB> bad;
+      Redo<RB, NB> bad;
       bad.find(acc);
       wait_vm0();  // the stores above are done
       __syncthreads();
@@ -1266,7 +1277,10 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
 // ((p0 + p1) + p2) + p3.  Each row's p_w is its own slots of residue w in
 // ascending order (a slot the row does not use adds exact zeros), so every
 // output is still a fixed sequence of fp32 operations, independent of which
-// rows share its tile.
+// rows share its tile.  f32 operands are split into three bf16 values by the
+// wave that loads them (each wave has weights of its own, so there is no slab
+// to split once): 64->64, 11k rows 47.4 us on the f32 unit, 35.8 this way;
+// 32->32, 25k rows 28.6 and 23.2.
 template <typename T, int BN, int CK>
 __global__ void __launch_bounds__(256, 2) conv_split_kernel(
     const T* __restrict__ feat, int c_in, const T* __restrict__ W, Epilogue ep,
@@ -1542,13 +1556,13 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
   if constexpr (!F32) {
     if (wave == 0) store(every);
   } else {
-    NonFinite<2, NB> bad;
+    Redo<2, NB> bad;
     if (wave == 0) {
       store(every);
       bad.find(acc);
     }
     // accumulators that are not finite once more on the f32 unit (above)
-    if (!__syncthreads_or(wave == 0 && NonFinite<2, NB>::any(acc))) return;
+    if (!__syncthreads_or(wave == 0 && Redo<2, NB>::any(acc))) return;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -1576,10 +1590,10 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
 //   * kSingle, feature buffers smaller than one piece: element by element.
 // C_out that is no multiple of 16 has zero-weight columns that are not stored.
 // These widths ran one row per lane on the vector ALU before, 20 class scores
-// with every feature row read by five column groups.  Per pass, before and
-// after: 96 -> 20 f16 over 120k rows 70 -> 21 us; a 3 -> 32 f16 layer with 125
-// slots over 80k rows, with its pair build, 209 -> 130 us; 5 -> 16 and 16 -> 16
-// f16 over 60k LiDAR rows, with the build, 90 -> 81 us.
+// with every feature row read by five column groups.  Before and after: 96 -> 20
+// f16 over 120k rows 70 -> 21 us a pass; a 3 -> 32 f16 layer with 125 slots over
+// 80k rows, its launch 121 -> 29 us; 5 -> 16 and 16 -> 16 f16 over 60k LiDAR
+// rows, a pass with the build 90 -> 81 us.
 // A group of steps loads all its map entries, then all its gathers and
 // weight operands, then runs its MFMAs, so a 3x3x3 layer with C_in = 4 (four
 // steps) costs two dependent memory round trips.  Each output is the same
