@@ -18,7 +18,8 @@ pytestmark = [pytest.mark.gpu, needs_gpu]
     (128, 128, torch.bfloat16, (51072, 51073)),   # 64 / 128 columns
     (64, 64, torch.float16, (131072, 131073)),    # 32 / 64 rows per wave
     (128, 128, torch.float16, (98304, 98305)),
-    (64, 64, torch.float32, (16384, 16385)),      # slot split / 32 columns
+    (64, 64, torch.float32, (20480, 20481)),      # slot split / 32 columns
+    (48, 64, torch.float32, (32768, 32769)),      # slot split / register gather
     (64, 64, torch.float32, (65408, 65409)),      # 32 / 64 columns
     (64, 64, torch.float32, (98304, 98305)),      # 32 / 64 rows per wave
     (48, 64, torch.float16, (20480, 20481)),      # slot split / register gather

@@ -1072,14 +1072,18 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   // f32 (split): the slab of s + 1 lands in the one load buffer, whose vectors
   // each wave splits into split slab S ^ 1 between wait 3 and the barrier; the
   // wait in 2 also covers those reads, so the slab of s + 2 may land there.
-  auto run = [&](auto split) {
+  // stages s (kc, cc), s + 1 (kn, cn) and s + 2 (kp, cp)
+  int kc, cc, kn, cn, kp, cp;
+  auto open = [&](auto split) {
     constexpr bool SPLIT = decltype(split)::value;
-    // stages s (kc, cc), s + 1 (kn, cn) and s + 2 (kp, cp)
-    int kc = -1, cc = nch - 1;
+    kc = -1;
+    cc = nch - 1;
     advance(kc, cc);
-    int kn = kc, cn = cc;
+    kn = kc;
+    cn = cc;
     advance(kn, cn);
-    int kp = kn, cp = cn;
+    kp = kn;
+    cp = cn;
     advance(kp, cp);
     if (kc < K) {
       dma_entries(0, kc);
@@ -1094,92 +1098,107 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
     dma_rows(0, cc, blocks(kc));
     wait_vm0();
     __syncthreads();
-
-    auto body = [&](auto slot) {
-      constexpr int S = decltype(slot)::value;
-      wait_vm0();
-      if (kn < K) dma_slab(SPLIT ? 0 : S ^ 1, kn, cn);
-      if (kp < K) dma_entries(S, kp);
-      const int cur = blocks(kc);
-      uint4 a[RB][UB];
+  };
+  auto body = [&](auto slot, auto split) {
+    constexpr int S = decltype(slot)::value;
+    constexpr bool SPLIT = decltype(split)::value;
+    wait_vm0();
+    if (kn < K) dma_slab(SPLIT ? 0 : S ^ 1, kn, cn);
+    if (kp < K) dma_entries(S, kp);
+    const int cur = blocks(kc);
+    uint4 a[RB][UB];
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        if ((cur >> rb) & 1) {
+    for (int rb = 0; rb < RB; ++rb) {
+      if ((cur >> rb) & 1) {
 #pragma unroll
-          for (int u = 0; u < UB; ++u) a[rb][u] = a_read(rb, u);
-        }
+        for (int u = 0; u < UB; ++u) a[rb][u] = a_read(rb, u);
       }
-      wait_lgkm0();
-      const int nxt = blocks(kn);
-      dma_rows(S ^ 1, cn, nxt);
-      // the MFMAs of the blocks that use slot kc (a wave-uniform branch per
-      // block; one loop, so the register allocation is that of a full wave)
-      if (SPLIT && cur) {
-        const uint4* sw = s_split + S * (SPLIT_BYTES / 16);
+    }
+    wait_lgkm0();
+    const int nxt = blocks(kn);
+    dma_rows(S ^ 1, cn, nxt);
+    // the MFMAs of the blocks that use slot kc (a wave-uniform branch per
+    // block; one loop, so the register allocation is that of a full wave)
+    if (SPLIT && cur) {
+      const uint4* sw = s_split + S * (SPLIT_BYTES / 16);
 #pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) {
-          Split8 as[RB];
+      for (int t2 = 0; t2 < 2; ++t2) {
+        Split8 as[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          if ((cur >> rb) & 1) as[rb] = split8(a[rb][2 * t2], a[rb][2 * t2 + 1]);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const Split8 b = load_split<NB>(sw, nb, t2, lane);
 #pragma unroll
           for (int rb = 0; rb < RB; ++rb)
-            if ((cur >> rb) & 1) as[rb] = split8(a[rb][2 * t2], a[rb][2 * t2 + 1]);
+            if ((cur >> rb) & 1) acc[rb][nb] = mfma_split(as[rb], b, acc[rb][nb]);
+        }
+      }
+    } else if (cur) {
+      const uint4* sw = s_w + S * SLAB_VECS;
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            const Split8 b = load_split<NB>(sw, nb, t2, lane);
+      for (int u = 0; u < UB; ++u) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const uint4 bv = sw[(nb * UB + u) * 64 + lane];
+          if constexpr (F32) {
+            // four 32x32x2 steps per vector: step e uses element e of A and B
+            const float4 b4 = __builtin_bit_cast(float4, bv);
+            const float bs[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int rb = 0; rb < RB; ++rb) {
+                if ((cur >> rb) & 1) {
+                  const float4 a4 = __builtin_bit_cast(float4, a[rb][u]);
+                  const float as[4] = {a4.x, a4.y, a4.z, a4.w};
+                  acc[rb][nb] = Op::run(as[e], bs[e], acc[rb][nb]);
+                }
+              }
+          } else {
+            const V b = __builtin_bit_cast(V, bv);
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
-              if ((cur >> rb) & 1) acc[rb][nb] = mfma_split(as[rb], b, acc[rb][nb]);
-          }
-        }
-      } else if (cur) {
-        const uint4* sw = s_w + S * SLAB_VECS;
-#pragma unroll
-        for (int u = 0; u < UB; ++u) {
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            const uint4 bv = sw[(nb * UB + u) * 64 + lane];
-            if constexpr (F32) {
-              // four 32x32x2 steps per vector: step e uses element e of A and B
-              const float4 b4 = __builtin_bit_cast(float4, bv);
-              const float bs[4] = {b4.x, b4.y, b4.z, b4.w};
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                  if ((cur >> rb) & 1) {
-                    const float4 a4 = __builtin_bit_cast(float4, a[rb][u]);
-                    const float as[4] = {a4.x, a4.y, a4.z, a4.w};
-                    acc[rb][nb] = Op::run(as[e], bs[e], acc[rb][nb]);
-                  }
-                }
-            } else {
-              const V b = __builtin_bit_cast(V, bv);
-#pragma unroll
-              for (int rb = 0; rb < RB; ++rb)
-                if ((cur >> rb) & 1)
-                  acc[rb][nb] = Op::run(__builtin_bit_cast(V, a[rb][u]), b, acc[rb][nb]);
-            }
+              if ((cur >> rb) & 1)
+                acc[rb][nb] = Op::run(__builtin_bit_cast(V, a[rb][u]), b, acc[rb][nb]);
           }
         }
       }
-      wait_rows(__builtin_popcount(nxt));
-      if constexpr (SPLIT) {
-        if (kn < K) split_slab(S ^ 1);
-      }
-      __syncthreads();
-      kc = kn;
-      cc = cn;
-      kn = kp;
-      cn = cp;
-      advance(kp, cp);
-    };
+    }
+    wait_rows(__builtin_popcount(nxt));
+    if constexpr (SPLIT) {
+      if (kn < K) split_slab(S ^ 1);
+    }
+    __syncthreads();
+    kc = kn;
+    cc = cn;
+    kn = kp;
+    cn = cp;
+    advance(kp, cp);
+  };
+  auto run = [&](auto split) {
+    open(split);
     while (kc < K) {
-      body(Slot<0>{});
-      body(Slot<1>{});
+      body(Slot<0>{}, split);
+      body(Slot<1>{}, split);
     }
     wait_vm0();
     __syncthreads();
   };
-  run(std::bool_constant<F32>{});
+  if constexpr (F32) {
+    run(std::true_type{});
+  } else {
+    // in place: through the lambda the compiler tests kc < K again in each
+    // stage (128->128 fp16, 500k rows 307 us in place, 311 so)
+    open(std::false_type{});
+    while (kc < K) {
+      body(Slot<0>{}, std::false_type{});
+      body(Slot<1>{}, std::false_type{});
+    }
+    wait_vm0();
+    __syncthreads();
+  }
   bool rerun = false;
   if constexpr (F32) rerun = __syncthreads_or(Redo<RB, NB>::any(acc));
 
@@ -1535,6 +1554,7 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
   auto store = [&](auto which) {
     const bool affine = ep.mean != nullptr;
     const bool relu = ep.relu != 0;
+    T* const dst = out + nbt * BN + (lane & 31);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -1546,7 +1566,7 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
         for (int nb = 0; nb < NB; ++nb) {
           const int cl = nb * 32 + (lane & 31);
           if (which(rb, nb, i))
-            out[(int64_t)orow * c_out + nbt * BN + cl] =
+            dst[(int64_t)orow * c_out + nb * 32] =
                 from_f32<T>(finish(acc[rb][nb][i] + s_bias[cl], s_scale[cl], s_shift[cl], affine, relu));
         }
       }
@@ -1554,7 +1574,8 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
   run(std::bool_constant<F32>{});
   auto every = [](int, int, int) { return true; };
   if constexpr (!F32) {
-    if (wave == 0) store(every);
+    if (wave != 0) return;
+    store(every);
   } else {
     Redo<2, NB> bad;
     if (wave == 0) {
@@ -1986,11 +2007,18 @@ int dma_per_cu(int dtype, int bn, int rb) {
 //     (64->64, 8k rows 14.1 against 15.7; 10k rows 18.5 against 15.9), two for
 //     a single column tile (inverse 64->32, 30k rows 15.2 against 17.1), for
 //     strided and inverse layers, whose rows use few slots (inverse 128->64,
-//     15k rows 21.4 against 27.8; strided 64->128, 6k rows 15.5 against 16.6), for
-//     K < 12 (32->64 with 8 slots, 20k rows 10.2 against 8.6) and for f32
-//     (64->64, 16k rows 48 against 50; 128->128, 16k rows 173 against 115), and
-//     two and a half for the other f16/bf16 layers (32->32, 28k rows 12.8
-//     against 15.7; 48->64, 20k rows 20.2 against 24.3, 28k 25.1 against 24.5).
+//     15k rows 21.4 against 27.8; strided 64->128, 6k rows 15.5 against 16.6) and
+//     for K < 12 (32->64 with 8 slots, 20k rows 10.2 against 8.6), and two and a
+//     half for the other f16/bf16 layers (32->32, 28k rows 12.8 against 15.7;
+//     48->64, 20k rows 20.2 against 24.3, 28k 25.1 against 24.5) and for f32
+//     (32->32, 40k rows 31.5 against 33.3, 50k 36.9 against 33.6; 64->64, 18k rows
+//     44.5 against 59.4; 128->128, 9k rows 76 against 113).  f32 strided and
+//     inverse layers and those of the register-gather kernel with more than one
+//     column tile up to four (inverse 128->64, 24k rows 36.4 against 46.0;
+//     48->96, 16k rows 44.6 against 65.9; 16->64, 32k rows 36.3 against 37.4).
+//     SubM layers of the direct-to-LDS kernel would gain up to five (64->64, 40k
+//     rows 72.9 against 78.4), but keep the 256-row kernels' sums, bit for bit,
+//     past two and a half: a 64->128 layer of 12k rows has always had them.
 //   * Rows per wave of the direct-to-LDS kernel: 32 (128-row tiles) below
 //     kShortTiles 256-row tiles, as halving a wave's rows halves each stage's
 //     MFMAs and the smaller pool lets more workgroups share a CU; but 64 where
@@ -2021,8 +2049,11 @@ MfmaChoice choose_mfma(int dtype, int c_in, int c_out, int K, int64_t n_in, int6
     return tiles(256) < (c.bn == 128 ? 360 : f32 || K < 12 ? 300 : 128);
   };
   while (c.bn > 32 && few()) c.bn /= 2;
-  const bool two = f32 || (dma ? c_out == 32 || n_in != n_out : K < 12);
-  const int64_t split_tiles = two ? 2 * kCus : dma ? kCus : 5 * kCus / 2;
+  const bool two = dma ? c_out == 32 || n_in != n_out : K < 12;
+  const int64_t split_tiles = f32   ? (c_out > 32 && (n_in != n_out || !dma) ? 4 * kCus : 5 * kCus / 2)
+                              : two ? 2 * kCus
+                              : dma ? kCus
+                                    : 5 * kCus / 2;
   c.split = c.bn == 32 && K >= 8 && tiles(kSplitRows) <= split_tiles;
   c.dma = dma && !c.split;
   if (c.dma && tiles(256) < kShortTiles) {
