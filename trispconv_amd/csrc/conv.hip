@@ -1612,7 +1612,7 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
 // C_out that is no multiple of 16 has zero-weight columns that are not stored.
 // These widths ran one row per lane on the vector ALU before, 20 class scores
 // with every feature row read by five column groups.  Before and after: 96 -> 20
-// f16 over 120k rows 70 -> 21 us a pass; a 3 -> 32 f16 layer with 125 slots over
+// f16 over 120k rows 70 -> 14 us a pass; a 3 -> 32 f16 layer with 125 slots over
 // 80k rows, its launch 121 -> 29 us; 5 -> 16 and 16 -> 16 f16 over 60k LiDAR
 // rows, a pass with the build 90 -> 81 us.
 // A group of steps loads all its map entries, then all its gathers and
