@@ -31,6 +31,7 @@
 // no folded copy of them can go stale.
 #include "common.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace tsc {
@@ -138,6 +139,18 @@ __device__ __forceinline__ float src_weight(const void* w, int dt, int layout, i
   return load_any(w, dt, idx);
 }
 
+// f32 layers of the 32x32 tile: the buffer's last float is a word about the
+// weights' range.  Where the last chunk is half padding (C_in % 32 == 16), that
+// float is padding, which only ever multiplies zero rows; the other layouts are
+// 16 bytes longer for it.  kNoSplit is a finite number, so its products with
+// zeros are zeros.
+constexpr uint32_t kNoSplit = 0xff7fffffu;        // -FLT_MAX, above every magnitude's bits
+constexpr uint32_t kSplitHolds = (127 - 110) << 23;  // 2^-110: larger values split without a rest
+__host__ __device__ __forceinline__ int range_tail(int c_in) { return c_in % 32 ? 0 : 4; }
+__host__ __device__ __forceinline__ uint32_t* range_word(const float* packed, int64_t layout, int c_in) {
+  return reinterpret_cast<uint32_t*>(const_cast<float*>(packed)) + layout + range_tail(c_in) - 1;
+}
+
 // MFMA layout: [k][chunk][c_out/32][u][lane][16/sizeof(T)].  Lane l of a
 // 32-column block n supplies column n*32 + l%32, and for lane half h = l/32
 // the channels c*CK + h*CK/2 + u*(16/sizeof(T)) + 0.. of chunk c: the same
@@ -169,6 +182,25 @@ __global__ void pack_mfma_kernel(const void* w, int w_dt, int layout, int K, int
     packed[e] = from_f32<T>(ci < c_in ? src_weight(w, w_dt, layout, K, c_in, c_out, k, ci, co)
                                       : 0.f);
   }
+  if constexpr (std::is_same<T, float>::value)  // the layout's range word (below), before its maximum
+    if (blockIdx.x == 0 && threadIdx.x == 0) *range_word(packed, total, c_in) = 0u;
+}
+
+// The range word of an f32 layer's packed weights: the bits of their largest
+// magnitude, or kNoSplit where a weight is not finite or so small that three
+// bf16 values do not hold it.  256 weights a block and step, one atomic per
+// wave.
+__global__ void __launch_bounds__(256) weight_range_kernel(const void* w, int w_dt, int64_t count,
+                                                           uint32_t* word) {
+  uint32_t most = 0;
+  for (int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x; e < count; e += (int64_t)gridDim.x * 256) {
+    const uint32_t v = __float_as_uint(load_any(w, w_dt, e)) & 0x7fffffffu;
+    const bool held = v < 0x7f800000u && (v == 0 || v >= kSplitHolds);
+    most = max(most, held ? v : kNoSplit);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) most = max(most, static_cast<uint32_t>(__shfl_xor(most, off, kWave)));
+  if ((threadIdx.x & 63) == 0) atomicMax(word, most);
 }
 
 // The direct-to-LDS kernel's output rows are written once and not read
@@ -257,12 +289,20 @@ template <> struct MfmaOp<float> {
 // 27 x 64 -> 64 SubM, 100k rows, 5.3e-7 and 4.5e-7; 64 -> 64 stride 2 on
 // LiDAR voxels 4.4e-7 and 3.7e-7.  Their times (the first's launch, the
 // second's whole frame with its build and plan): 179 -> 133 us, 301 -> 251 us.
-// A value that is not finite or rounds to infinity in bf16 makes its products
-// NaN, and below 2^-109 lo runs out of bf16's exponents (an absolute error of
-// up to 2^-126, were such numbers flushed).  The accumulators that end up not
-// finite or below 2^-80 without being zero are computed once more on the f32
-// unit (Redo below), so such outputs are what that unit gives; in the others
-// 27 x 64 errors of 2^-126 are below 2^-35 of the sum.
+// What three bf16 values cannot hold is computed once more on the f32 unit
+// (Redo below), element by element, so that neither the tile nor the order
+// decides which sums those are:
+//   * A value that is not finite or rounds to infinity in bf16 makes its
+//     products NaN: accumulators that end up not finite.
+//   * Below 2^-110 lo is short of bf16's exponents (subnormals, which both units
+//     keep, end at 2^-133): an error of up to 2^-134, times the other operand.
+//     For features that is at most max|w| 2^-134 for each of up to 2^18
+//     products, so sums of at least max|w| 2^-88 have it below 2^-28 of them,
+//     and smaller ones are computed again (max|w| from the range word of the
+//     packed weights).  A sum of exactly zero is, where its row gathers a value
+//     so small that all three parts may vanish.
+//   * Layers with such weights run on the f32 unit throughout: nothing bounds
+//     the features that would multiply their errors.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
@@ -323,17 +363,47 @@ __device__ __forceinline__ Split8 load_split(const uint4* slab, int nb, int t, i
   return {plane(0), plane(1), plane(2)};
 }
 
-// The elements of this lane's accumulators that the f32 unit computes again:
-// not finite, or too small for the split (0 < |x| < 2^-80).  One bit each.
+// The smallest sum that the split settles, from the packed weights' range word;
+// infinity: none (the layer runs on the f32 unit).
+__device__ __forceinline__ float split_limit(uint32_t range) {
+  const float limit = fmaxf(0x1p-80f, __uint_as_float(range) * 0x1p-88f);
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(
+      range == kNoSplit ? 0x7f800000u : __float_as_uint(limit)));
+}
+
+// Bit r set: row r of a 32-row block is in `rows` and gathers a value other than
+// zero below 2^-132, which the split may turn into nothing.  s_orow: the block's
+// output rows; first: its first processing position.
+__device__ uint32_t vanishing_rows(const float* __restrict__ feat, int c_in,
+                                   const int32_t* __restrict__ nbr, int nbr_ordered, int64_t n_out,
+                                   int K, const int32_t* s_orow, int64_t first, uint32_t rows) {
+  constexpr uint32_t kVanishing = (1u << 17) << 1;  // 2^-132's bits, shifted left
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int32_t o = s_orow[r];
+  bool any = false;
+  if (o >= 0 && ((rows >> r) & 1)) {
+    for (int k = 0; k < K; ++k) {
+      const int32_t j = nbr ? nbr[(int64_t)k * n_out + (nbr_ordered ? first + r : (int64_t)o)] : o;
+      if (j < 0) continue;
+      const uint4* src = reinterpret_cast<const uint4*>(feat + (int64_t)j * c_in);
+      for (int c = h; c < c_in / 4; c += 2) {
+        const uint4 v = src[c];
+        for (const uint32_t x : {v.x, v.y, v.z, v.w}) any |= (x << 1) - 1u < kVanishing - 1u;
+      }
+    }
+  }
+  const uint64_t b = __ballot(any);
+  return static_cast<uint32_t>(b) | static_cast<uint32_t>(b >> 32);
+}
+
+// The elements of this lane's accumulators that the f32 unit computes again (see
+// above), one bit each.
 template <int RB, int NB>
 struct Redo {
-  static constexpr uint32_t kSmall = 47u << 24;  // 2^-80's bits without the sign, shifted left
   uint32_t bits[(RB * NB + 1) / 2];
-  // whether there are any: 0 * x is 0 for every finite x, else NaN; a zero
-  // passes the other check, as the largest value
-  static __device__ __forceinline__ bool any(const f32x16 (&acc)[RB][NB]) {
-    float z = 0.f;
-    uint32_t least = 0xffffffffu;
+  // whether there may be any: 0 * x is 0 for every finite x, else NaN
+  static __device__ __forceinline__ bool any(const f32x16 (&acc)[RB][NB], float limit) {
+    float z = 0.f, least = 3.4028235e38f;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -341,11 +411,42 @@ struct Redo {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           z = fmaf(acc[rb][nb][i], 0.f, z);
-          least = min(least, (__float_as_uint(acc[rb][nb][i]) << 1) - 1u);
+          least = fminf(least, fabsf(acc[rb][nb][i]));
         }
-    return !(z == 0.f) || least < kSmall - 1u;
+    return !(z == 0.f) || least < limit;
   }
-  __device__ __forceinline__ void find(const f32x16 (&acc)[RB][NB]) {
+  // a wave's rows past the layer's last (it has `left` rows) sum to 1, not 0: a
+  // layer's partial tile would otherwise always look for vanished sums, at the
+  // end of the launch (64->64, 100k rows 132 -> 137 us)
+  static __device__ __forceinline__ void pad(f32x16 (&acc)[RB][NB], int64_t left) {
+    if (left >= 32 * RB) return;
+    const int h = (threadIdx.x & 63) >> 5;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (rb * 32 + (i >> 2) * 8 + h * 4 + (i & 3) >= left) acc[rb][nb][i] = 1.f;
+  }
+  // rows of block rb with an element of exactly zero, as row bits
+  static __device__ __forceinline__ uint32_t zero_rows(const f32x16 (&acc)[NB]) {
+    uint32_t rows = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      bool zero = false;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) zero |= acc[nb][i] == 0.f;
+      const uint64_t b = __ballot(zero);
+      const int r = (i >> 2) * 8 + (i & 3);
+      rows |= (static_cast<uint32_t>(b) ? 1u << r : 0u) | (static_cast<uint32_t>(b >> 32) ? 16u << r : 0u);
+    }
+    return rows;
+  }
+  // vanish: per block, the rows whose zeros may be sums that vanished
+  __device__ __forceinline__ void find(const f32x16 (&acc)[RB][NB], float limit,
+                                       const uint32_t (&vanish)[RB]) {
+    const int h = (threadIdx.x & 63) >> 5;
     for (uint32_t& b : bits) b = 0;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
@@ -353,11 +454,21 @@ struct Redo {
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const uint32_t v = __float_as_uint(acc[rb][nb][i]) << 1;
-          const bool bad = v >= 0xff000000u || v - 1u < kSmall - 1u;
+          const float v = fabsf(acc[rb][nb][i]);
+          const int r = (i >> 2) * 8 + h * 4 + (i & 3);
+          const bool bad = !(v <= 3.4028235e38f) ||
+                           (v < limit && (v != 0.f || ((vanish[rb] >> r) & 1)));
           const int e = (rb * NB + nb) * 16 + i;
           bits[e / 32] |= (bad ? 1u : 0u) << (e % 32);
         }
+  }
+  __device__ __forceinline__ void all() {
+    for (uint32_t& b : bits) b = 0xffffffffu;
+  }
+  __device__ __forceinline__ bool some() const {
+    uint32_t m = 0;
+    for (const uint32_t b : bits) m |= b;
+    return m != 0;
   }
   __device__ __forceinline__ bool has(int rb, int nb, int i) const {
     const int e = (rb * NB + nb) * 16 + i;
@@ -432,6 +543,8 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   const int64_t tile0 = static_cast<int64_t>(item / ncol) * kTileRows;
   const int nbt = static_cast<int>(item % ncol);
   const int nch = (c_in + CK - 1) / CK;  // C_in % 16 == 0: the last chunk may be half padding
+  uint32_t range = 0;  // f32: asked for here, used after the set-up
+  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in);
 
   // ---- tile set-up: output rows, their slot lists and slot masks.  The map
   // entries are read 32 slots at a time, all in flight before any is used
@@ -540,6 +653,7 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[rb][nb][i] = 0.f;
+  if constexpr (F32) Redo<2, NB>::pad(acc, n_out - tile0 - wave * 64);
 
   uint4 ring[RING][2][UB];  // gathered operands: this stage and the next
   uint4 w0, w1, w2, w3;        // this thread's share of the next weight slab
@@ -639,6 +753,9 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
     }
   };
 
+  const float limit = F32 ? split_limit(range) : 0.f;
+  const bool no_split = F32 && limit > 3.4028235e38f;  // the f32 unit computes the whole tile, below
+
   // Two waves per SIMD (two workgroups per CU): while one wave waits for its
   // gathers or at the barrier, the other's MFMAs keep the matrix core busy.
   // The next stage's loads are issued before this stage's MFMAs, the weights
@@ -653,6 +770,7 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
     advance(kn, cn);
     load_w(kc, cc);
     load_a(Slot<0>{}, kc, cc);
+    if (decltype(split)::value && no_split) kc = K;  // here, so that the first loads do not wait for it
     store_w(s_w[0], split);
     __syncthreads();
     auto body = [&](auto slot) {
@@ -674,7 +792,7 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   };
   run(std::bool_constant<F32>{});
   bool rerun = false;
-  if constexpr (F32) rerun = __syncthreads_or(Redo<2, NB>::any(acc));
+  if constexpr (F32) rerun = __syncthreads_or(Redo<2, NB>::any(acc, limit));
 
   // ---- epilogue: + bias (and the affine map and ReLU when asked), round
   // once, store each output element once.
@@ -702,6 +820,7 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   }
 #pragma unroll
   for (int pass = 0; pass < 64 / PR; ++pass) {
+    if (no_split) break;
     __syncthreads();                                // the staging area is free
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
@@ -740,7 +859,21 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   if constexpr (F32) {
     if (rerun) {  // workgroup-uniform, and rare
       Redo<2, NB> bad;
-      bad.find(acc);
+      if (no_split) {
+        bad.all();
+      } else {
+        uint32_t vanish[2];
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+          const uint32_t zeros = Redo<2, NB>::zero_rows(acc[rb]);
+          vanish[rb] = zeros ? vanishing_rows(feat, c_in, nbr, nbr_ordered, n_out, K,
+                                              s_orow + wave * 64 + rb * 32, tile0 + wave * 64 + rb * 32,
+                                              zeros)
+                             : 0u;
+        }
+        bad.find(acc, limit, vanish);
+      }
+      if (!__syncthreads_or(bad.some())) return;
       // the stores above are done, and the staged slot lists are read again
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -857,6 +990,8 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   const int64_t tile0 = static_cast<int64_t>(item / ncol) * TR;
   const int nbt = static_cast<int>(item % ncol);
   const int nch = c_in / CK;
+  uint32_t range = 0;
+  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in);
 
   // ---- tile set-up: output rows and slot masks (the entries themselves are
   // loaded again stage by stage), as in conv_mfma_kernel; thread t < TR
@@ -1060,6 +1195,7 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[rb][nb][i] = 0.f;
+  if constexpr (F32) Redo<RB, NB>::pad(acc, n_out - tile0 - wave * WR);
 
   // Stage s (slab and entry buffers S = s % 2), with the three waits:
   //  1. vmcnt(0): this wave's rows of s have landed (issued in stage s - 1);
@@ -1073,6 +1209,8 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   // each wave splits into split slab S ^ 1 between wait 3 and the barrier; the
   // wait in 2 also covers those reads, so the slab of s + 2 may land there.
   // stages s (kc, cc), s + 1 (kn, cn) and s + 2 (kp, cp)
+  const float limit = F32 ? split_limit(range) : 0.f;
+  const bool no_split = F32 && limit > 3.4028235e38f;  // the f32 unit computes the whole tile, below
   int kc, cc, kn, cn, kp, cp;
   auto open = [&](auto split) {
     constexpr bool SPLIT = decltype(split)::value;
@@ -1098,6 +1236,7 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
     dma_rows(0, cc, blocks(kc));
     wait_vm0();
     __syncthreads();
+    if (SPLIT && no_split) kc = K;  // here, so that the first loads do not wait for it
   };
   auto body = [&](auto slot, auto split) {
     constexpr int S = decltype(slot)::value;
@@ -1200,7 +1339,7 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
     __syncthreads();
   }
   bool rerun = false;
-  if constexpr (F32) rerun = __syncthreads_or(Redo<RB, NB>::any(acc));
+  if constexpr (F32) rerun = __syncthreads_or(Redo<RB, NB>::any(acc, limit));
 
   // ---- epilogue, as in conv_mfma_kernel, staged in the pool
   const bool affine = ep.mean != nullptr;
@@ -1224,6 +1363,7 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   }
 #pragma unroll
   for (int pass = 0; pass < WR / PR; ++pass) {
+    if (no_split) break;
     __syncthreads();
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
@@ -1262,7 +1402,21 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   if constexpr (F32) {
     if (rerun) {  // workgroup-uniform, and rare
       Redo<RB, NB> bad;
-      bad.find(acc);
+      if (no_split) {
+        bad.all();
+      } else {
+        uint32_t vanish[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+          const uint32_t zeros = Redo<RB, NB>::zero_rows(acc[rb]);
+          vanish[rb] = zeros ? vanishing_rows(feat, c_in, nbr, nbr_ordered, n_out, K,
+                                              s_orow + wave * WR + rb * 32, tile0 + wave * WR + rb * 32,
+                                              zeros)
+                             : 0u;
+        }
+        bad.find(acc, limit, vanish);
+      }
+      if (!__syncthreads_or(bad.some())) return;
       wait_vm0();  // the stores above are done
       __syncthreads();
 #pragma unroll
@@ -1331,6 +1485,8 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
   const int64_t tile0 = static_cast<int64_t>(item / ncol) * SR;
   const int nbt = static_cast<int>(item % ncol);
   const int nch = (c_in + CK - 1) / CK;
+  uint32_t range = 0;
+  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in);
 
   // ---- set-up: wave w reads the map entries of its own slots for the 64
   // rows, sixteen slots at a time, all in flight before any is used; a map
@@ -1425,6 +1581,7 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[rb][nb][i] = 0.f;
+  if constexpr (F32) Redo<2, NB>::pad(acc, n_out - tile0);
 
   uint4 ring[2][2][UB];   // gathered operands: this stage and the next
   uint4 bring[2][NB][UB];  // weight operands: this stage and the next
@@ -1505,6 +1662,8 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
     }
   };
 
+  const float limit = F32 ? split_limit(range) : 0.f;
+  const bool no_split = F32 && limit > 3.4028235e38f;  // the f32 unit computes the whole tile, below
   auto run = [&](auto split) {
     int kc = -1, cc = nch - 1;
     advance(kc, cc);  // this wave's first slot
@@ -1512,6 +1671,7 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
     advance(kn, cn);
     load_b(Slot<0>{}, kc, cc);
     load_a(Slot<0>{}, kc, cc);
+    if (decltype(split)::value && no_split) kc = K;  // here, so that the first loads do not wait for it
     auto body = [&](auto slot) {
       constexpr int S = decltype(slot)::value;
       load_b(Slot<(S + 1) % 2>{}, kn, cn);  // next stage's weights
@@ -1571,19 +1731,30 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
         }
       }
   };
-  run(std::bool_constant<F32>{});
   auto every = [](int, int, int) { return true; };
   if constexpr (!F32) {
+    run(std::false_type{});
     if (wave != 0) return;
     store(every);
   } else {
+    run(std::true_type{});
+    if (wave == 0 && !no_split) store(every);
+    if (!__syncthreads_or(wave == 0 && Redo<2, NB>::any(acc, limit))) return;
     Redo<2, NB> bad;
-    if (wave == 0) {
-      store(every);
-      bad.find(acc);
+    if (no_split) {
+      bad.all();
+    } else if (wave == 0) {
+      uint32_t vanish[2];
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        const uint32_t zeros = Redo<2, NB>::zero_rows(acc[rb]);
+        vanish[rb] = zeros ? vanishing_rows(feat, c_in, nbr, nbr_ordered, n_out, K, s_orow + rb * 32,
+                                            tile0 + rb * 32, zeros)
+                           : 0u;
+      }
+      bad.find(acc, limit, vanish);
     }
-    // accumulators that are not finite once more on the f32 unit (above)
-    if (!__syncthreads_or(wave == 0 && Redo<2, NB>::any(acc))) return;
+    if (!__syncthreads_or(wave == 0 && bad.some())) return;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -2185,7 +2356,8 @@ extern "C" int64_t tsc_packed_weight_bytes(int32_t k_vol, int32_t c_in, int32_t 
                                            int32_t dtype) {
   if (pick_path(dtype, c_in, c_out, k_vol) == kMfma) {
     const int ck = pick_ck(dtype, c_in);
-    return (int64_t)k_vol * mfma_chunks(c_in, ck) * ck * c_out * dtype_bytes(dtype);
+    return ((int64_t)k_vol * mfma_chunks(c_in, ck) * ck * c_out +
+            (dtype == TSC_F32 ? range_tail(c_in) : 0)) * dtype_bytes(dtype);
   }
   const int64_t bytes = narrow_steps(dtype, k_vol, c_in) * ceil_div(c_out, 16) * 64 * 16;
   // widths that do not fill their pieces and tiles: no less than an fp32
@@ -2218,10 +2390,13 @@ extern "C" int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, i
           w, w_dtype, layout, k_vol, c_in, c_out, nsteps, static_cast<__hip_bfloat16*>(packed));
   } else if (path == kMfma) {
     const int ck = pick_ck(dtype, c_in);
-    if (dtype == TSC_F32)
-      pack_mfma_kernel<float><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out, ck,
-                                                   static_cast<float*>(packed));
-    else if (dtype == TSC_F16)
+    if (dtype == TSC_F32) {
+      float* const p = static_cast<float*>(packed);
+      pack_mfma_kernel<float><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out, ck, p);
+      const int64_t count = (int64_t)k_vol * c_in * c_out;
+      weight_range_kernel<<<static_cast<unsigned>(std::min<int64_t>(ceil_div(count, 1024), 1024)), 256, 0, s>>>(
+          w, w_dtype, count, range_word(p, (int64_t)k_vol * mfma_chunks(c_in, ck) * ck * c_out, c_in));
+    } else if (dtype == TSC_F16)
       pack_mfma_kernel<__half><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out, ck,
                                                     static_cast<__half*>(packed));
     else
