@@ -26,9 +26,8 @@
 // to 32 slots), which the mask pass writes: one 128-byte row per position
 // instead of one scattered entry per slot.
 //
-// Sorting: stable LSD radix passes with 9-bit digits; with one region, one pass
-// on the mask's leading nine bits and a sort of each bucket in LDS
-// (bucket_sort_kernel).  Each pass is a histogram kernel (per-block digit counts,
+// Sorting: stable LSD radix passes with 9-bit digits (a 27-slot mask sorts
+// in three passes).  Each pass is a histogram kernel (per-block digit counts,
 // digit-major), a scan of each digit's counts over the blocks (one workgroup
 // per digit) and a stable scatter, whose blocks add the digits' bases
 // themselves and in which each wave ranks equal digits with nine ballots.  The first sort
@@ -37,7 +36,6 @@
 // region (position / region_rows).
 #include "common.hpp"
 
-#include <algorithm>
 #include <utility>
 
 namespace tsc {
@@ -452,148 +450,6 @@ __global__ void __launch_bounds__(kRadix) small_sort_kernel(const uint32_t* __re
   }
 }
 
-// Columns that one 9-bit digit pass has put in order of their masks' leading
-// bits, brought into the order of the whole mask, stably: a workgroup takes up
-// to kChunk columns of one leading-bits bucket and sorts them by the low_bits
-// bits below in LDS, each word a column's low mask bits over its place in the
-// chunk (kChunkBits bits).  A bucket of more than kChunk columns is sorted chunk
-// by chunk, in the order it has, which for raster columns keeps each chunk's
-// rows near each other: its tiles' masks repeat per chunk.  One launch instead
-// of the two further passes' six; per digit pass, each wave counts its share
-// of the words, one scan gives every (digit, wave) its first place, and the waves then
-// place their words, 64 at a time, without a barrier.  Measured against the two
-// passes: 166k LiDAR rows 23.7 us against 30.7 and five launches fewer, the
-// layer's frame 256 -> 238 us; 500k surface rows 37 against 39 us, two layers'
-// frame 824 -> 821.  A workgroup's latency is its chunk's rounds: chunks of 7680
-// in 512 threads took 39 and 45 us.
-constexpr int kChunkBits = 13;
-constexpr int kChunk = 5120;
-constexpr int kChunkThreads = 1024;
-constexpr int kChunkWaves = kChunkThreads / kWave;
-static_assert(kChunk <= 1 << kChunkBits, "a place in the chunk has kChunkBits bits");
-constexpr size_t kChunkLds = (2 * kChunk + kChunkWaves * kRadix) * sizeof(uint32_t);
-static_assert(kRadix <= kChunkThreads, "a thread per digit");
-
-__global__ void __launch_bounds__(kChunkThreads) bucket_sort_kernel(
-    const uint32_t* __restrict__ vals_in, const uint32_t* __restrict__ mask_pos,
-    const uint32_t* __restrict__ digit_tot, int low_bits, uint32_t* __restrict__ vals_out) {
-  extern __shared__ uint32_t s_chunk[];
-  uint32_t* src = s_chunk;
-  uint32_t* dst = s_chunk + kChunk;
-  uint32_t* s_base = s_chunk + 2 * kChunk;  // [wave][digit]
-  __shared__ uint32_t s_wave[33];
-  __shared__ uint32_t s_start, s_len;
-  const int t = threadIdx.x, w = t / kWave, lane = t & (kWave - 1);
-  {  // which bucket's which chunk this workgroup takes
-    if (t == 0) s_len = 0;
-    const uint32_t c = t < kRadix ? digit_tot[t] : 0u;
-    const uint32_t chunks = (c + kChunk - 1) / kChunk;
-    uint32_t tot;
-    const uint32_t start = block_exclusive(c, s_wave, &tot);
-    const uint32_t first = block_exclusive(chunks, s_wave, &tot);
-    if (blockIdx.x >= first && blockIdx.x < first + chunks) {
-      const uint32_t skip = (blockIdx.x - first) * kChunk;
-      s_start = start + skip;
-      s_len = c - skip < static_cast<uint32_t>(kChunk) ? c - skip : kChunk;
-    }
-    __syncthreads();
-  }
-  const int len = static_cast<int>(s_len);
-  if (len == 0) return;  // more workgroups than chunks
-  const int64_t start = s_start;
-  const uint32_t low = (1u << low_bits) - 1u;
-  // kBatch columns of a thread have their loads in flight together (indexes
-  // past the chunk read its first column)
-  constexpr int kBatch = 4;
-  for (int i0 = t; i0 < len; i0 += kBatch * kChunkThreads) {
-    uint32_t v[kBatch];
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int i = i0 + j * kChunkThreads;
-      v[j] = vals_in[start + (i < len ? i : 0)];
-    }
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) v[j] = mask_pos[v[j]];
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int i = i0 + j * kChunkThreads;
-      if (i < len) src[i] = (v[j] & low) << kChunkBits | static_cast<uint32_t>(i);
-    }
-  }
-  uint32_t* const base = s_base + w * kRadix;
-  // whole rounds of 64 words per wave, in wave order
-  const int share = ((len + kChunkWaves - 1) / kChunkWaves + kWave - 1) / kWave * kWave;
-  const int w_lo = w * share < len ? w * share : len;
-  const int w_hi = w_lo + share < len ? w_lo + share : len;
-  for (int shift = kChunkBits; shift < kChunkBits + low_bits; shift += kDigitBits) {
-    for (int r = t; r < kChunkWaves * kRadix; r += kChunkThreads) s_base[r] = 0;
-    __syncthreads();
-    for (int i0 = w_lo; i0 < w_hi; i0 += kWave) {
-      const int i = i0 + lane;
-      const bool valid = i < w_hi;
-      const uint32_t dg = valid ? (src[i] >> shift) & (kRadix - 1u) : 0u;
-      // one add where the wave's words share a digit, as a large bucket's do
-      const uint32_t d0 = __builtin_amdgcn_readfirstlane(dg);
-      const uint64_t words = __ballot(valid);  // by the whole wave
-      if (__ballot(valid && dg != d0) == 0ull) {
-        if (lane == 0) atomicAdd(&base[d0], static_cast<uint32_t>(__popcll(words)));
-      } else if (valid) {
-        atomicAdd(&base[dg], 1u);
-      }
-    }
-    __syncthreads();
-    uint32_t sum = 0;
-    if (t < kRadix)
-      for (int ww = 0; ww < kChunkWaves; ++ww) sum += s_base[ww * kRadix + t];
-    uint32_t tot;
-    uint32_t run = block_exclusive(sum, s_wave, &tot);
-    if (t < kRadix)
-      for (int ww = 0; ww < kChunkWaves; ++ww) {
-        const uint32_t c = s_base[ww * kRadix + t];
-        s_base[ww * kRadix + t] = run;
-        run += c;
-      }
-    __syncthreads();
-    for (int i0 = w_lo; i0 < w_hi; i0 += kWave) {
-      const int i = i0 + lane;
-      const bool valid = i < w_hi;
-      const uint32_t word = valid ? src[i] : 0u;
-      const uint32_t dg = (word >> shift) & (kRadix - 1u);
-      uint64_t peers = __ballot(valid);
-#pragma unroll
-      for (int b = 0; b < kDigitBits; ++b) {
-        const uint64_t ones = __ballot((dg >> b) & 1u);
-        peers &= ((dg >> b) & 1u) ? ones : ~ones;
-      }
-      const int rank = rank_in_wave(peers);
-      const uint32_t at = base[dg] + rank;  // read by every lane before the first of them adds
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      if (valid) {
-        if (rank == 0) base[dg] += static_cast<uint32_t>(__popcll(peers));
-        if (at < static_cast<uint32_t>(kChunk)) dst[at] = word;  // holds by construction
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    }
-    __syncthreads();
-    uint32_t* const other = src;
-    src = dst;
-    dst = other;
-  }
-  for (int i0 = t; i0 < len; i0 += kBatch * kChunkThreads) {
-    uint32_t v[kBatch];
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int i = i0 + j * kChunkThreads;
-      v[j] = vals_in[start + (src[i < len ? i : 0] & ((1u << kChunkBits) - 1u))];
-    }
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int i = i0 + j * kChunkThreads;
-      if (i < len) vals_out[start + i] = v[j];
-    }
-  }
-}
-
 struct Buffers {
   uint32_t *keys_a, *keys_b, *vals_a, *vals_b, *rows, *mask_pos, *hist, *hist_off, *digit_tot;
   int32_t* nbr_t;  // the map's row-major copy (K <= 32), else null
@@ -728,27 +584,17 @@ extern "C" int tsc_conv_plan(const int32_t* nbr, const int32_t* cols_row, int32_
   const int mask_bits = k_vol < 32 ? k_vol : 32;
   const int64_t regions = ceil_div(n_out, region_rows);
   const int region_bits = bits_for(static_cast<uint64_t>(regions - 1));
-  const int low_bits = mask_bits - kDigitBits;
-  if (regions == 1 && low_bits > 0 && low_bits + kChunkBits <= 32) {
-    // leading bits first, then each bucket by the rest in LDS
-    const Digits d{kFromMaskAtValue, low_bits, nullptr, b.mask_pos, 1u};
+  // All of the mask, digit by digit.  One pass on the leading nine bits and each
+  // bucket's rest in LDS takes 7 us less on 165k LiDAR rows (23.7 against 30.7,
+  // a new frame 242 against 252), but a workgroup's LDS holds 5k columns, and a
+  // larger bucket is then sorted in pieces, whose tiles meet more masks.  Slots
+  // of all 256-row tiles, so against fully sorted: 500k surface rows 36,747 and
+  // 35,617, those LiDAR rows 7,083 and 6,525, a plane of 120k voxels, which is
+  // one bucket, 3,114 and 1,940; every convolution over the order pays for them.
+  for (int p = 0; p < (mask_bits + kDigitBits - 1) / kDigitBits; ++p) {
+    const Digits d{kFromMaskAtValue, kDigitBits * p, nullptr, b.mask_pos, 1u};
     if ((rc = radix_pass(b, nullptr, vi, nullptr, vo, n_out, d, s))) return rc;
     std::swap(vi, vo);
-    if ((rc = allow_dynamic_lds(reinterpret_cast<const void*>(&bucket_sort_kernel),
-                                static_cast<int>(kChunkLds))))
-      return rc;
-    // at most one partial chunk per bucket
-    const int64_t chunks = n_out / kChunk + std::min<int64_t>(kRadix, n_out);
-    bucket_sort_kernel<<<static_cast<unsigned>(chunks), kChunkThreads, kChunkLds, s>>>(
-        vi, b.mask_pos, b.digit_tot, low_bits, vo);
-    TSC_LAUNCH_CHECK("plan_bucket_sort");
-    std::swap(vi, vo);
-  } else {
-    for (int p = 0; p < (mask_bits + kDigitBits - 1) / kDigitBits; ++p) {
-      const Digits d{kFromMaskAtValue, kDigitBits * p, nullptr, b.mask_pos, 1u};
-      if ((rc = radix_pass(b, nullptr, vi, nullptr, vo, n_out, d, s))) return rc;
-      std::swap(vi, vo);
-    }
   }
   for (int p = 0; p < (region_bits + kDigitBits - 1) / kDigitBits; ++p) {
     const Digits d{kFromRegionOfValue, kDigitBits * p, nullptr, nullptr,
