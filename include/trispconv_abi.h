@@ -339,7 +339,10 @@ TSC_API int tsc_map_masks(const int32_t* nbr, int64_t n, int32_t k_vol, int32_t*
  *                     (the internal (K, C_in, C_out) layout, and the 1x1x1
  *                      fold quirk, which re-reads KRSC storage this way)
  * The packed layout and size depend on (k_vol, c_in, c_out, dtype), which
- * choose the convolution kernel; pack once per such tuple.
+ * choose the convolution kernel; pack once per such tuple.  Weights of another
+ * type than dtype are rounded to it, except for 16-bit features and widths with
+ * c_in % 4 != 0 or c_out % 16 != 0, which multiply the weights' own values in
+ * fp32 (such a layer runs far below the speed of weights of its own type).
  * ------------------------------------------------------------------------ */
 TSC_API int64_t tsc_packed_weight_bytes(int32_t k_vol, int32_t c_in, int32_t c_out, int32_t dtype);
 TSC_API int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, int32_t k_vol, int32_t c_in,

@@ -227,6 +227,36 @@ __device__ __forceinline__ void store_out(void* dst, uint4 v, bool nt) {
 // their loads (64 bytes per lane are read at most).
 __device__ __attribute__((aligned(256))) uint4 g_zero_row[16];
 
+// Weights of widths that do not fill the narrow kernel's pieces and tiles keep
+// their own type: packed for 16-bit features they come in one of two forms, told
+// apart by the buffer's last word.
+//   * Weights of the features' type: the narrow layout, and kNarrowForm (a NaN
+//     with bits of its own).
+//   * Others: f32, [slot][channel][column].  The last word is then the last
+//     weight, with a NaN's bits made plain, or 0 in a longer buffer.
+constexpr uint32_t kNarrowForm = 0x7fc5a51eu;
+bool has_forms(int dtype, int c_in, int c_out) {
+  return dtype != TSC_F32 && (c_in % 4 != 0 || c_out % 16 != 0);
+}
+int64_t narrow_bytes(int dtype, int K, int c_in, int c_out) {
+  return narrow_steps(dtype, K, c_in) * ceil_div(c_out, 16) * 64 * 16;
+}
+
+__global__ void __launch_bounds__(256) pack_wide_kernel(const void* w, int w_dt, int layout, int K,
+                                                        int c_in, int c_out, float* packed,
+                                                        uint32_t* form) {
+  const int64_t total = (int64_t)K * c_in * c_out;
+  for (int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
+    const int co = e % c_out;
+    const int ci = (e / c_out) % c_in;
+    const int k = e / ((int64_t)c_in * c_out);
+    const float v = src_weight(w, w_dt, layout, K, c_in, c_out, k, ci, co);
+    packed[e] = v == v ? v : __uint_as_float(0x7fc00000u);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0 && form >= reinterpret_cast<uint32_t*>(packed) + total)
+    *form = 0u;
+}
+
 // Narrow layout: [step i][ceil(c_out/16)][lane][LV], LV = 16 / sizeof(T)
 // values.  Lane l of 16-column tile n supplies column n*16 + l%16 and the
 // reduction values r = 4*LV*i + LV*(l/16) + 0..LV-1, r = k * cp + c for slot k
@@ -235,7 +265,8 @@ __device__ __attribute__((aligned(256))) uint4 g_zero_row[16];
 // channel and the last column.
 template <typename T>
 __global__ void pack_narrow_kernel(const void* w, int w_dt, int layout, int K, int c_in,
-                                   int c_out, int64_t nsteps, T* packed) {
+                                   int c_out, int64_t nsteps, T* packed, uint32_t* form) {
+  if (form && blockIdx.x == 0 && threadIdx.x == 0) *form = kNarrowForm;
   constexpr int LV = 16 / (int)sizeof(T);
   const int nt_all = (c_out + 15) / 16;
   const int cp = (c_in + 3) / 4 * 4;
@@ -1842,8 +1873,8 @@ __device__ __forceinline__ uint4 join_pieces(const uint16_t* v) {
                     v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
 }
 
-// Four channels read at the byte address p, of which the first `bytes - shift`
-// bytes after `shift` are wanted: shifted into place, the rest cleared.
+// Four channels read at the byte address p: shifted down by `shift` bytes, of
+// which the first `bytes` are wanted and the rest cleared.
 __device__ __forceinline__ uint2 ragged_piece(const char* p, uint32_t shift, uint32_t bytes,
                                               uint2) {
   uint64_t v;
@@ -1906,9 +1937,10 @@ constexpr int kBufferWord3 = 0x00020000;  // raw buffer, 32-bit data (gfx9 famil
 
 template <typename T, int READ, int PIECE, int NT, bool B32>
 __global__ void __launch_bounds__(256) conv_narrow_kernel(
-    const T* __restrict__ feat, int64_t feat_bytes, int c_in, const T* __restrict__ W, Epilogue ep,
-    const int32_t* __restrict__ nbr, const int32_t* __restrict__ order, int nbr_ordered,
-    int64_t n_out, int K, int c_out, int nsteps, NarrowB32 nb32, T* __restrict__ out) {
+    const T* __restrict__ feat, int64_t feat_bytes, int c_in, const T* __restrict__ W,
+    const uint32_t* __restrict__ form, Epilogue ep, const int32_t* __restrict__ nbr,
+    const int32_t* __restrict__ order, int nbr_ordered, int64_t n_out, int K, int c_out, int nsteps,
+    NarrowB32 nb32, T* __restrict__ out) {
   using Op = Mfma16<T>;
   using Piece = typename VecOf<PIECE>::type;
   constexpr int LV = 16 / (int)sizeof(T);      // reduction values per lane and step
@@ -1937,6 +1969,9 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
   const Piece* zero_piece =
       (const Piece*)reinterpret_cast<const __attribute__((address_space(1))) Piece*>(zero_addr);
   const uint4* Wv = reinterpret_cast<const uint4*>(W);
+  // the weights' form, asked for here and used at the end: the main loop over
+  // f32 weights reads inside the buffer too, and its sums are dropped
+  const uint32_t form_word = sizeof(T) == 2 && form ? *form : kNarrowForm;
 
   // the epilogue's per-column parameters: loaded before the main loop (their
   // latency overlaps the map loads), combined after it
@@ -2048,6 +2083,33 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
       const uint4 a = join_pieces(v + u * NP);
 #pragma unroll
       for (int n = 0; n < NT; ++n) acc[n] = Op::step(a, b[u][n], acc[n]);
+    }
+  }
+
+  // f32 weights under 16-bit features (rare: a program packs weights of the
+  // features' type): each output's products one by one in f32, slots and channels
+  // ascending
+  if (sizeof(T) == 2 && form_word != kNarrowForm) {
+    const float* const wf = reinterpret_cast<const float*>(W);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int64_t p = p0 + 4 * q + e;
+      const int64_t o = p < n_out ? (order ? order[p] : p) : 0;
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[n][e] = 0.f;
+      for (int k = 0; k < K && p < n_out; ++k) {
+        const int64_t j = nbr ? nbr[(int64_t)k * n_out + (nbr_ordered ? p : o)] : o;
+        if (j < 0) continue;
+        for (int c = 0; c < c_in; ++c) {
+          const float x = to_f32<T>(feat[j * c_in + c]);
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            const int co = (nt0 + n) * 16 + rl;
+            acc[n][e] = fmaf(x, wf[((int64_t)k * c_in + c) * c_out + (co < c_out ? co : c_out - 1)],
+                             acc[n][e]);
+          }
+        }
+      }
     }
   }
 
@@ -2279,6 +2341,9 @@ int launch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, const
   TSC_REQUIRE(nsteps < (int64_t(1) << 26), "conv: K * C_in too large");
   constexpr int elem = static_cast<int>(sizeof(T));
   const int64_t feat_bytes = n_in * c_in * elem;
+  const uint32_t* form = nullptr;
+  if (has_forms(dt, c_in, c_out))
+    form = reinterpret_cast<const uint32_t*>(W) + tsc_packed_weight_bytes(K, c_in, c_out, dt) / 4 - 1;
   const int64_t cols = ceil_div(c_out, 16) / NT;
   TSC_REQUIRE(cols < 65536, "conv: C_out too large");
   dim3 grid(static_cast<unsigned>(ceil_div(n_out, 4 * kNarrowRows)), static_cast<unsigned>(cols));
@@ -2289,11 +2354,11 @@ int launch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, const
                          static_cast<uint32_t>(c_in * elem),
                          static_cast<uint32_t>(((uint64_t(1) << 32) + cp - 1) / cp)};
     conv_narrow_kernel<T, READ, PIECE, NT, true><<<grid, 256, 0, s>>>(
-        static_cast<const T*>(feat), feat_bytes, c_in, static_cast<const T*>(W), ep, nbr, order,
+        static_cast<const T*>(feat), feat_bytes, c_in, static_cast<const T*>(W), form, ep, nbr, order,
         nbr_ordered, n_out, K, c_out, static_cast<int>(nsteps), nb32, static_cast<T*>(out));
   } else {
     conv_narrow_kernel<T, READ, PIECE, NT, false><<<grid, 256, 0, s>>>(
-        static_cast<const T*>(feat), feat_bytes, c_in, static_cast<const T*>(W), ep, nbr, order,
+        static_cast<const T*>(feat), feat_bytes, c_in, static_cast<const T*>(W), form, ep, nbr, order,
         nbr_ordered, n_out, K, c_out, static_cast<int>(nsteps), NarrowB32{}, static_cast<T*>(out));
   }
   TSC_LAUNCH_CHECK("conv_narrow");
@@ -2333,8 +2398,14 @@ int dispatch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, con
   if (read == kRagged && n_in * c_in * elem < ragged) read = kSingle;
   const int piece = read == kWhole ? whole : read == kRagged ? ragged : elem;
   if (read == kSingle) nt = 1;
-#define TSC_NARROW_CASE(R_, P_, NT_)                                                            if (read == R_ && piece == P_ && nt == NT_)                                                     return launch_narrow<T, R_, P_, NT_>(feat, n_in, c_in, W, ep, nbr, order, nbr_ordered,                                             n_out, K, c_out, out, s);
-#define TSC_NARROW_CASES(R_, P_)   TSC_NARROW_CASE(R_, P_, 1) TSC_NARROW_CASE(R_, P_, 2) TSC_NARROW_CASE(R_, P_, 3) \
+#define TSC_NARROW_CASE(R_, P_, NT_)                                                         \
+  if (read == R_ && piece == P_ && nt == NT_)                                                \
+    return launch_narrow<T, R_, P_, NT_>(feat, n_in, c_in, W, ep, nbr, order, nbr_ordered,   \
+                                         n_out, K, c_out, out, s);
+#define TSC_NARROW_CASES(R_, P_)                                                             \
+  TSC_NARROW_CASE(R_, P_, 1)                                                                 \
+  TSC_NARROW_CASE(R_, P_, 2)                                                                 \
+  TSC_NARROW_CASE(R_, P_, 3)                                                                 \
   TSC_NARROW_CASE(R_, P_, 4)
   TSC_NARROW_CASES(kWhole, 16)
   if constexpr (sizeof(T) == 2) {
@@ -2359,11 +2430,13 @@ extern "C" int64_t tsc_packed_weight_bytes(int32_t k_vol, int32_t c_in, int32_t 
     return ((int64_t)k_vol * mfma_chunks(c_in, ck) * ck * c_out +
             (dtype == TSC_F32 ? range_tail(c_in) : 0)) * dtype_bytes(dtype);
   }
-  const int64_t bytes = narrow_steps(dtype, k_vol, c_in) * ceil_div(c_out, 16) * 64 * 16;
+  const int64_t bytes = narrow_bytes(dtype, k_vol, c_in, c_out);
   // widths that do not fill their pieces and tiles: no less than an fp32
-  // (K, C_in, C_out) copy, the size these weights have always had
+  // (K, C_in, C_out) copy, the size these weights have always had, and for
+  // 16-bit features a word past the narrow layout for the form
   const int64_t fp32 = (int64_t)k_vol * c_in * c_out * 4;
-  return (c_in % 4 || c_out % 16) && fp32 > bytes ? fp32 : bytes;
+  if ((c_in % 4 || c_out % 16) && fp32 > bytes) return fp32;
+  return bytes + (has_forms(dtype, c_in, c_out) ? 16 : 0);
 }
 
 extern "C" int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, int32_t k_vol,
@@ -2379,15 +2452,21 @@ extern "C" int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, i
   const Path path = pick_path(dtype, c_in, c_out, k_vol);
   if (path == kNarrow) {
     const int64_t nsteps = narrow_steps(dtype, k_vol, c_in);
-    if (dtype == TSC_F32)
-      pack_narrow_kernel<float><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out,
-                                                     nsteps, static_cast<float*>(packed));
+    uint32_t* form = nullptr;
+    if (has_forms(dtype, c_in, c_out))
+      form = static_cast<uint32_t*>(packed) + tsc_packed_weight_bytes(k_vol, c_in, c_out, dtype) / 4 - 1;
+    if (form && w_dtype != dtype)
+      pack_wide_kernel<<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out,
+                                            static_cast<float*>(packed), form);
+    else if (dtype == TSC_F32)
+      pack_narrow_kernel<float><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out, nsteps,
+                                                     static_cast<float*>(packed), form);
     else if (dtype == TSC_F16)
-      pack_narrow_kernel<__half><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out,
-                                                      nsteps, static_cast<__half*>(packed));
+      pack_narrow_kernel<__half><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out, nsteps,
+                                                      static_cast<__half*>(packed), form);
     else
-      pack_narrow_kernel<__hip_bfloat16><<<grid, 256, 0, s>>>(
-          w, w_dtype, layout, k_vol, c_in, c_out, nsteps, static_cast<__hip_bfloat16*>(packed));
+      pack_narrow_kernel<__hip_bfloat16><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out, nsteps,
+                                                              static_cast<__hip_bfloat16*>(packed), form);
   } else if (path == kMfma) {
     const int ck = pick_ck(dtype, c_in);
     if (dtype == TSC_F32) {
