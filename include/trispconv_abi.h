@@ -182,8 +182,14 @@ TSC_API int tsc_pairs_from_map(const int32_t* nbr, int64_t n, int32_t k_vol, int
                                void* ws, int64_t ws_bytes, int32_t* pairs_in,
                                int32_t* pairs_out, tsc_stream_t stream);
 /* The reference's int64 lists from padded tables [K][cap]: the first sizes[k]
- * (0..cap) entries of every slot k, one slot after the other, in pairs_in and
- * pairs_out order.  lists_in and lists_out hold the sum of the sizes. */
+ * (0..cap) entries of every slot k.  _each: into memory of their own, lists_in[k]
+ * and lists_out[k] (host arrays of device addresses; either array may be NULL,
+ * and an address whose slot is empty).  tsc_pair_lists: one slot after the
+ * other, lists_in and lists_out holding the sum of the sizes. */
+TSC_API int tsc_pair_lists_each(const int32_t* pairs_in, const int32_t* pairs_out, int32_t k_vol,
+                                int64_t cap, const int64_t* sizes /* host, [K] */,
+                                int64_t* const* lists_in /* host, [K] */,
+                                int64_t* const* lists_out /* host, [K] */, tsc_stream_t stream);
 TSC_API int tsc_pair_lists(const int32_t* pairs_in, const int32_t* pairs_out, int32_t k_vol,
                            int64_t cap, const int64_t* sizes /* host, [K] */, int64_t* lists_in,
                            int64_t* lists_out, tsc_stream_t stream);

@@ -49,6 +49,8 @@ _SIGNATURES = {
     "tsc_map_to_rows": (ctypes.c_int, [_vp, _vp, _i64, _i64, _i32, _vp, _vp]),
     "tsc_pairs_from_map_workspace_bytes": (_i64, [_i64, _i32]),
     "tsc_pairs_from_map": (ctypes.c_int, [_vp, _i64, _i32, _i64, _vp, _i64, _vp, _vp, _vp]),
+    "tsc_pair_lists_each": (ctypes.c_int, [_vp, _vp, _i32, _i64, ctypes.POINTER(_i64),
+                                           ctypes.POINTER(_vp), ctypes.POINTER(_vp), _vp]),
     "tsc_pair_lists": (ctypes.c_int, [_vp, _vp, _i32, _i64, ctypes.POINTER(_i64), _vp, _vp, _vp]),
     "tsc_strided_workspace_bytes": (_i64, [_i64, _i32, _i32, c_i32p, _i32]),
     "tsc_strided_marks_bytes": (_i64, [_i64, _i32, _i32, c_i32p]),

@@ -1087,33 +1087,33 @@ __global__ void __launch_bounds__(kRows) subm_fill_kernel(const int32_t* __restr
   }
 }
 
-// The int64 lists of up to kListSlots slots from the padded int32 tables, one
-// slot after the other: off[k] is where slot k's list starts.  The offsets come
-// by value, so no copy of the host's counts to the device is waited for.  A
-// thread converts kListItems entries a block apart, so loads and stores stay
-// whole lines.  All lists of a build in one launch, where each slot's two lists
-// were a torch copy each: a pass that makes the lists of a 100k-voxel
-// submanifold build, a strided one and its inverse, 86 lists in all, 777 -> 331
-// us (7.0 us of it the 54 submanifold lists' launch).
+// The int64 lists of up to kListSlots slots from the padded int32 tables, each
+// into memory of its own (null: that list is not wanted).  Sizes and addresses
+// come by value, so no copy of the host's to the device is waited for.  A thread
+// converts kListItems entries a block apart, so loads and stores stay whole
+// lines.  All lists of a build in one launch (7.0 us for the 54 of a 100k-voxel
+// submanifold build), where each list was a torch copy.
 constexpr int kListSlots = 64;
 constexpr int kListItems = 4;
-struct ListOffsets {
-  int64_t off[kListSlots + 1];
+struct ListSlots {
+  int64_t size[kListSlots];
+  int64_t* in[kListSlots];
+  int64_t* out[kListSlots];
 };
 __global__ void __launch_bounds__(256) pair_lists_kernel(const int32_t* __restrict__ pairs_in,
                                                          const int32_t* __restrict__ pairs_out,
-                                                         int64_t cap, ListOffsets o,
-                                                         int64_t* __restrict__ lists_in,
-                                                         int64_t* __restrict__ lists_out) {
+                                                         int64_t cap, ListSlots lists) {
   const int k = blockIdx.y;
-  const int64_t base = o.off[k], size = o.off[k + 1] - base;
+  const int64_t size = lists.size[k];
+  int64_t* const in = lists.in[k];
+  int64_t* const out = lists.out[k];
   const int64_t first = blockIdx.x * (int64_t)(256 * kListItems) + threadIdx.x;
 #pragma unroll
   for (int q = 0; q < kListItems; ++q) {
     const int64_t i = first + q * 256;
     if (i >= size) return;
-    lists_in[base + i] = pairs_in[(int64_t)k * cap + i];
-    lists_out[base + i] = pairs_out[(int64_t)k * cap + i];
+    if (in) in[i] = pairs_in[(int64_t)k * cap + i];
+    if (out) out[i] = pairs_out[(int64_t)k * cap + i];
   }
 }
 
@@ -1640,33 +1640,63 @@ extern "C" int tsc_pairs_from_map(const int32_t* nbr, int64_t n, int32_t k_vol, 
   return 0;
 }
 
-extern "C" int tsc_pair_lists(const int32_t* pairs_in, const int32_t* pairs_out, int32_t k_vol,
-                              int64_t cap, const int64_t* sizes, int64_t* lists_in,
-                              int64_t* lists_out, tsc_stream_t stream) {
+extern "C" int tsc_pair_lists_each(const int32_t* pairs_in, const int32_t* pairs_out, int32_t k_vol,
+                                   int64_t cap, const int64_t* sizes, int64_t* const* lists_in,
+                                   int64_t* const* lists_out, tsc_stream_t stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   TSC_REQUIRE(k_vol > 0 && cap >= 0 && cap < (int64_t(1) << 31) && sizes,
               "pair_lists: invalid sizes");
-  for (int32_t k = 0; k < k_vol; ++k)
+  for (int32_t k = 0; k < k_vol; ++k) {
     TSC_REQUIRE(sizes[k] >= 0 && sizes[k] <= cap, "pair_lists: slot %d has %lld of %lld entries",
                 static_cast<int>(k), static_cast<long long>(sizes[k]), static_cast<long long>(cap));
-  int64_t at = 0;
+    TSC_REQUIRE(sizes[k] == 0 || ((!lists_in || (pairs_in && lists_in[k])) &&
+                                  (!lists_out || (pairs_out && lists_out[k]))),
+                "pair_lists: null pointer");
+  }
   for (int32_t k0 = 0; k0 < k_vol; k0 += kListSlots) {
     const int slots = static_cast<int>(std::min<int32_t>(kListSlots, k_vol - k0));
-    ListOffsets o;
+    ListSlots l{};
     int64_t most = 0;
-    o.off[0] = at;
     for (int k = 0; k < slots; ++k) {
-      most = std::max(most, sizes[k0 + k]);
-      o.off[k + 1] = at += sizes[k0 + k];
+      l.size[k] = sizes[k0 + k];
+      l.in[k] = lists_in ? lists_in[k0 + k] : nullptr;
+      l.out[k] = lists_out ? lists_out[k0 + k] : nullptr;
+      most = std::max(most, l.size[k]);
     }
     if (most == 0) continue;
-    TSC_REQUIRE(pairs_in && pairs_out && lists_in && lists_out, "pair_lists: null pointer");
     const dim3 grid(static_cast<unsigned>(ceil_div(most, 256 * kListItems)),
                     static_cast<unsigned>(slots));
     pair_lists_kernel<<<grid, 256, 0, s>>>(pairs_in + (int64_t)k0 * cap,
-                                           pairs_out + (int64_t)k0 * cap, cap, o, lists_in,
-                                           lists_out);
+                                           pairs_out + (int64_t)k0 * cap, cap, l);
     TSC_LAUNCH_CHECK("pair_lists");
+  }
+  return 0;
+}
+
+extern "C" int tsc_pair_lists(const int32_t* pairs_in, const int32_t* pairs_out, int32_t k_vol,
+                              int64_t cap, const int64_t* sizes, int64_t* lists_in,
+                              int64_t* lists_out, tsc_stream_t stream) {
+  TSC_REQUIRE(k_vol > 0 && cap >= 0 && cap < (int64_t(1) << 31) && sizes,
+              "pair_lists: invalid sizes");
+  int64_t total = 0;
+  for (int32_t k = 0; k < k_vol; ++k) {
+    TSC_REQUIRE(sizes[k] >= 0 && sizes[k] <= cap, "pair_lists: slot %d has %lld of %lld entries",
+                static_cast<int>(k), static_cast<long long>(sizes[k]), static_cast<long long>(cap));
+    total += sizes[k];
+  }
+  if (total == 0) return 0;
+  TSC_REQUIRE(pairs_in && pairs_out && lists_in && lists_out, "pair_lists: null pointer");
+  int64_t at = 0;
+  for (int32_t k0 = 0; k0 < k_vol; k0 += kListSlots) {
+    const int32_t slots = std::min<int32_t>(kListSlots, k_vol - k0);
+    int64_t *in[kListSlots], *out[kListSlots];
+    for (int32_t k = 0; k < slots; at += sizes[k0 + k++]) {
+      in[k] = lists_in + at;
+      out[k] = lists_out + at;
+    }
+    if (int rc = tsc_pair_lists_each(pairs_in + (int64_t)k0 * cap, pairs_out + (int64_t)k0 * cap, slots,
+                                     cap, sizes + k0, in, out, stream))
+      return rc;
   }
   return 0;
 }
