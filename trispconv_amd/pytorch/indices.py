@@ -111,8 +111,8 @@ class IndiceData:
         # reading them on the build's stream, or None);
         # counts[K] holds the build's status flags
         self._counts_pending: Optional[Tuple[torch.Tensor, int, Optional[Callable[[], None]]]] = None
-        # a strided build's counts on the host ([K + 3], a ctypes array), from
-        # which pair_num is made when it is read
+        # a strided build's counts on the host ([K + 3] numbers), from which
+        # pair_num is made when it is read
         self._host_counts = None
         self._pairs_in = pairs_in
         self._pairs_out = pairs_out
@@ -147,7 +147,7 @@ class IndiceData:
         # strided builds: each input row's id among the rows with a pair (-1
         # for the others), the inverse's output ids
         self._in_ids: Optional[torch.Tensor] = None
-        # and their geometry as ABI arguments
+        # and their kernel, stride, padding and dilation as they were built
         self._geo: Optional[tuple] = None
         # input rows the pairs may name: ids lie in [0, _in_bound) (the
         # builders' input rows; for user-assigned lists their largest id + 1)
@@ -849,10 +849,10 @@ def generate_strided_indice_pairs(indices: torch.Tensor, spatial_shape, batch_si
         output_spatial_shape=out_shape, kernel_size=ks, stride=st, padding=pd, dilation=dil,
         subm=False, pin=pin, pout=pout, cnt_dev=counts[:K], pair_num=None, nbr=nbr,
         batch_size=int(batch_size), rows_raster=True)
-    data._host_counts = host
+    data._host_counts = host[:]  # plain numbers: the ctypes array would not pickle
     data._n_in_paired = host[K + 2]
     data._in_ids = tables[o_ids:o_ids + n]
-    data._geo = sz.geo
+    data._geo = (ks, st, pd, dil)
     _STRIDED_BITMAPS[out_coords] = (ws, sz.out_words, tuple(out_shape), int(batch_size),
                                     out_coords._version,
                                     (out_coords.data_ptr(), out_coords.storage_offset()))
@@ -911,22 +911,23 @@ def _group_inverse(fwd: IndiceData, n_out: int, channel_work: int) -> bool:
     """Whether the inverse of ``fwd`` gets its columns grouped by the slots they
     can use: strides that leave more than one residue class, and a layer that
     skips unused slots (``channel_work`` > 0, see inverse_pairs_for)."""
-    st = fwd.stride
+    st = fwd.stride if fwd._geo is None else fwd._geo[1]
     return fwd._geo is not None and 1 < st[0] * st[1] * st[2] <= 64 \
         and 2 * n_out * fwd.K * channel_work >= _GROUP_MIN_WORK
 
 
 @functools.lru_cache(maxsize=64)
-def _grouped_ws_bytes(n_in: int, stride) -> int:
-    return int(L.lib().tsc_inverse_grouped_workspace_bytes(n_in, L.i3(stride)))
+def _grouped_sizes(n_in: int, geo) -> tuple:
+    """(workspace bytes, kernel, stride, padding and dilation as ABI arguments)."""
+    args = tuple(L.i3(v) for v in geo)
+    return (int(L.lib().tsc_inverse_grouped_workspace_bytes(n_in, args[1])), *args)
 
 
 def _grouped_inverse(fwd: IndiceData, in_coords: torch.Tensor, n_out: int, stream) -> IndiceData:
     """The inverse of a strided build made here, its map by grouped columns."""
     lib, dev, K, n_in = L.lib(), fwd._pin.device, fwd.K, len(fwd.input_indices)
     cap = fwd._pin.shape[1]
-    _, ks, st, pd, dil, _ = fwd._geo
-    ws_bytes = _grouped_ws_bytes(n_in, fwd.stride)
+    ws_bytes, ks, st, pd, dil = _grouped_sizes(n_in, fwd._geo)
     ws = L.workspace(ws_bytes, dev)
     out_coords = torch.empty((n_out, 4), dtype=torch.int32, device=dev)
     # cols_row, the map with room for its slot masks as row K, the pair table
