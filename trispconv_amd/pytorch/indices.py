@@ -898,21 +898,30 @@ def _strided_sizes(n, batch_size, shape, ks, st, pd, dil, out_shape) -> _Strided
 
 # A convolution over an inverse map in row order runs nearly every slot for
 # every tile; over grouped columns, only those its rows have.  Grouping takes
-# two more launches, so it is done where the former is some 40 us or more of
-# matrix work: multiply-adds over all slots times 2, f32 ones counted three
-# times (the rate such layers reach: 250 TFLOP/s f16, 85 f32).  Measured, down
-# and up again on new voxels: 128->64 f32, 8.5k rows 231 -> 186 us; 64->32
-# bf16, 250k rows (27e9) 196 -> 177; 60k rows (6.6e9), where the host's time
-# hides the convolution, 128 -> 152.
-_GROUP_MIN_WORK = 10_000_000_000
+# two more launches and some 10 us of host time, so it is done where the former
+# is enough matrix work to show behind a frame's host time: multiply-adds over
+# all slots times 2, f32 ones counted four times.  Measured, down and up again
+# on new voxels, row order and grouped, us:
+#   64->32 f16/bf16: 90k rows (10e9) 119 / 132, 130k (14e9) 134 / 148, 160k
+#     (18e9) 137 / 146, 200k (22e9) 155 / 145, 350k (39e9) 217 / 191
+#   128->64: 16k (7e9) 107 / 124, 25k (11e9) 126 / 123, 32k (14e9) 130 / 131,
+#     45k (20e9) 137 / 133, 80k (35e9) 163 / 145
+#   256->128: 5k (9e9) 132 / 143, 8k (14e9) 137 / 145, 14k (25e9) 183 / 158
+#   f32 64->32: 30k (13e9) 132 / 137, 50k (22e9) 172 / 148; 128->64: 8k (14e9)
+#     136 / 147, 10k (18e9) 155 / 147, 12k (21e9) 152 / 143
+#   2x2x2, 128->64 bf16: 150k (20e9) 126 / 137, 200k (26e9) 143 / 146, 300k
+#     (39e9) 153 / 145; f32 64->32: 150k (20e9) 142 / 145, 250k (33e9) 164 / 143
+_GROUP_MIN_WORK = 20_000_000_000
 
 
 def _group_inverse(fwd: IndiceData, n_out: int, channel_work: int) -> bool:
     """Whether the inverse of ``fwd`` gets its columns grouped by the slots they
     can use: strides that leave more than one residue class, and a layer that
     skips unused slots (``channel_work`` > 0, see inverse_pairs_for)."""
-    st = fwd.stride if fwd._geo is None else fwd._geo[1]
-    return fwd._geo is not None and 1 < st[0] * st[1] * st[2] <= 64 \
+    if fwd._geo is None:
+        return False
+    st = fwd._geo[1]
+    return 1 < st[0] * st[1] * st[2] <= 64 \
         and 2 * n_out * fwd.K * channel_work >= _GROUP_MIN_WORK
 
 
@@ -957,7 +966,7 @@ def inverse_pairs_for(fwd: IndiceData, c_in: int, c_out: int, dtype: torch.dtype
     computed in ``dtype``: the same pairs, their map laid out for it."""
     # the 32x32-tile kernels skip unused slots, the narrow one runs them all
     tiled = c_in % 16 == 0 and c_out % 32 == 0 and fwd.K <= 64
-    work = c_in * c_out * (3 if dtype == torch.float32 else 1) if tiled else 0
+    work = c_in * c_out * (4 if dtype == torch.float32 else 1) if tiled else 0
     return _inverse_pairs(fwd, work)
 
 
