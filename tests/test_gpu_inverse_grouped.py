@@ -41,8 +41,14 @@ def test_grouped_columns_hold_the_row_order_map(k, s, p, d, n, monkeypatch):
     runs = cls[np.concatenate([[True], cls[1:] != cls[:-1]])]
     assert len(runs) == len(np.unique(runs))  # each class in one run
     assert all((np.diff(rows[cls == v]) > 0).all() for v in runs)  # rows ascend within it
+    # the slots of a class: per axis, the kernel offsets that land on its residue
+    ks, dil = np.array(g.kernel_size), np.array(g.dilation)
+    hits = [[sum(o * dil[a] % st[a] == r for o in range(ks[a])) for r in range(st[a])] for a in range(3)]
+    slots = [np.prod([hits[a][r] for a, r in enumerate(np.unravel_index(v, st))]) for v in runs]
+    say("classes", len(runs), slots)
+    assert (np.diff(slots) <= 0).all()
     most = np.array([int((got._map_cols >= 0).sum(0).cpu().numpy()[cls == v].max()) for v in runs])
-    say("classes", len(runs), most.tolist())
+    assert (most <= slots).all()
 
 
 @pytest.mark.parametrize("n", [300, 9000, 60000])
