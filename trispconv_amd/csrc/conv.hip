@@ -1969,9 +1969,7 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
   const Piece* zero_piece =
       (const Piece*)reinterpret_cast<const __attribute__((address_space(1))) Piece*>(zero_addr);
   const uint4* Wv = reinterpret_cast<const uint4*>(W);
-  // the weights' form, asked for here and used at the end: the main loop over
-  // f32 weights reads inside the buffer too, and its sums are dropped
-  const uint32_t form_word = sizeof(T) == 2 && form ? *form : kNarrowForm;
+  uint32_t form_word = kNarrowForm;  // the weights' form: the buffer's last word
 
   // the epilogue's per-column parameters: loaded before the main loop (their
   // latency overlaps the map loads), combined after it
@@ -2077,6 +2075,16 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
         b[u][n] = i0 + u < nsteps
                       ? load_words(Wv + ((int64_t)(i0 + u) * nt_all + nt0 + n) * 64 + lane)
                       : make_uint4(0u, 0u, 0u, 0u);
+    if constexpr (sizeof(T) == 2) {
+      // Behind the group's loads, which it then shares the wait with; it is used
+      // after the loop, whose sums over f32 weights (reads inside the buffer
+      // too) are dropped.  Loaded at the kernel's start it is waited for with the
+      // kernel's other scalars: 96 -> 20, 120k rows 13.95 -> 14.3 us a pass, 14.0
+      // so.  The barrier keeps the compiler from moving it there.
+      const uint32_t* f = form;
+      asm volatile("" : "+s"(f));
+      form_word = *f;
+    }
 #pragma unroll
     for (int u = 0; u < SG; ++u) {
       if (i0 + u >= nsteps) break;
@@ -2089,7 +2097,7 @@ __global__ void __launch_bounds__(256) conv_narrow_kernel(
   // f32 weights under 16-bit features (rare: a program packs weights of the
   // features' type): each output's products one by one in f32, slots and channels
   // ascending
-  if (sizeof(T) == 2 && form_word != kNarrowForm) {
+  if (sizeof(T) == 2 && (c_in % 4 || c_out % 16) && form_word != kNarrowForm) {
     const float* const wf = reinterpret_cast<const float*>(W);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -2341,9 +2349,9 @@ int launch_narrow(const void* feat, int64_t n_in, int c_in, const void* W, const
   TSC_REQUIRE(nsteps < (int64_t(1) << 26), "conv: K * C_in too large");
   constexpr int elem = static_cast<int>(sizeof(T));
   const int64_t feat_bytes = n_in * c_in * elem;
-  const uint32_t* form = nullptr;
+  const uint32_t* form = static_cast<const uint32_t*>(W);  // read, and not looked at, where there is one form
   if (has_forms(dt, c_in, c_out))
-    form = reinterpret_cast<const uint32_t*>(W) + tsc_packed_weight_bytes(K, c_in, c_out, dt) / 4 - 1;
+    form += tsc_packed_weight_bytes(K, c_in, c_out, dt) / 4 - 1;
   const int64_t cols = ceil_div(c_out, 16) / NT;
   TSC_REQUIRE(cols < 65536, "conv: C_out too large");
   dim3 grid(static_cast<unsigned>(ceil_div(n_out, 4 * kNarrowRows)), static_cast<unsigned>(cols));
