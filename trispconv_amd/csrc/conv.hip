@@ -2258,8 +2258,9 @@ int dma_per_cu(int dtype, int bn, int rb) {
 //     column tile up to four (inverse 128->64, 24k rows 36.4 against 46.0;
 //     48->96, 16k rows 44.6 against 65.9; 16->64, 32k rows 36.3 against 37.4).
 //     SubM layers of the direct-to-LDS kernel would gain up to five (64->64, 40k
-//     rows 72.9 against 78.4), but keep the 256-row kernels' sums, bit for bit,
-//     past two and a half: a 64->128 layer of 12k rows has always had them.
+//     rows 72.9 against 78.4); their line is not where the times cross, but below
+//     the 752 tiles of a 64->128 layer of 12k rows, whose sums a test compares
+//     bit for bit with the 256-row kernels'.
 //   * Rows per wave of the direct-to-LDS kernel: 32 (128-row tiles) below
 //     kShortTiles 256-row tiles, as halving a wave's rows halves each stage's
 //     MFMAs and the smaller pool lets more workgroups share a CU; but 64 where

@@ -902,10 +902,9 @@ extern "C" int tsc_strided_fill(const int32_t* coords, int64_t n, int32_t batch_
 // kernel, which runs once the counts are there, stores them into pinned host
 // words, and the host spins on the word behind them while the fill still runs:
 // no copy, event or stream wait of their own.  The separate calls with a pinned
-// copy and an event between them took 73 us of host time per build in the
-// four-resolution fp16 encoder, this one 58: its pass over new voxels 830 -> 772
-// us, alternating on one machine, a 64->64 fp32 LiDAR frame 303 -> 248 with its
-// convolution's own gains.
+// copy and an event between them took 76-77 us of host time per build in the
+// four-resolution fp16 encoder, this one 59-63 (three alternations of processes
+// on one machine), its pass over new voxels 832-846 and 779-816 us.
 extern "C" int tsc_strided_build(const int32_t* coords, int64_t n, int32_t batch_size,
                                  const int32_t spatial[3], const int32_t ksize[3],
                                  const int32_t stride[3], const int32_t padding[3],
