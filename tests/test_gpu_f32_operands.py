@@ -8,6 +8,7 @@ from test_gpu_conv import _conv_raw, _module, _tiny
 from test_gpu_f32_split import _exact
 from trispconv_amd import _lib as L
 from trispconv_amd.pytorch.indices import generate_subm_indice_pairs
+from trispconv_amd.pytorch.weight import pack_weight
 
 pytestmark = [pytest.mark.gpu, needs_gpu]
 
@@ -76,6 +77,30 @@ def test_rows_of_small_values_among_ordinary_ones(c_in, c_out, n, grid, tile):
     keep = ordinary & ~sees(small)
     assert torch.equal(a[keep], b[keep])
     _check(a[only], _exact(mixed, m, nbr)[only])
+
+
+@pytest.mark.parametrize("c_in,c_out", [(64, 64), (48, 96), (16, 32)])
+@pytest.mark.parametrize("layout", ["krsc", "flat"])
+def test_dead_columns_and_vanishing_rows(c_in, c_out, layout):
+    """Columns without a weight stay zero while their rows' subnormal features
+    count in the others; one column has its only weight in the last slot."""
+    nbr, feats, m = _layer(c_in, c_out, 9000, 48, 1e-43, 1e30)
+    n = len(feats)
+    with torch.no_grad():
+        m.weight[[0, 5, c_out - 1]] = 0
+        m.weight[7] = 0
+        m.weight[7, 2, 2, 2, c_in - 1] = 3e29
+    w = m.weight.detach()
+    pw = m._packed_weight(torch.float32)
+    if layout == "flat":
+        flat = w.reshape(c_out, 27, c_in).permute(1, 2, 0).contiguous()
+        pw = pack_weight(flat, (27, 1, 1), c_in, c_out, torch.float32)
+    out = _conv_raw(feats, pw, m.bias, nbr, None, 0, n, 0)
+    ref = _exact(feats, m, nbr)
+    assert (out[:, [0, 5, c_out - 1]] == 0).all()
+    _check(out, ref)
+    _check(out[:, 7], ref[:, 7])
+    assert ((out == 0) == (ref == 0)).all()
 
 
 def test_zero_weights_and_zero_rows_give_zeros():

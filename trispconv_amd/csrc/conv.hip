@@ -139,16 +139,28 @@ __device__ __forceinline__ float src_weight(const void* w, int dt, int layout, i
   return load_any(w, dt, idx);
 }
 
-// f32 layers of the 32x32 tile: the buffer's last float is a word about the
-// weights' range.  Where the last chunk is half padding (C_in % 32 == 16), that
-// float is padding, which only ever multiplies zero rows; the other layouts are
-// 16 bytes longer for it.  kNoSplit is a finite number, so its products with
-// zeros are zeros.
+// f32 layers of the 32x32 tile hold two things about their weights besides them,
+// where the last chunk is half padding (C_in % 32 == 16) in that padding, which
+// only ever multiplies zero rows, else behind the layout:
+//   * the range word, the buffer's last: the bits of their largest magnitude, or
+//     kNoSplit where a weight is not finite or so small that three bf16 values
+//     do not hold it (a finite number, so its products with zeros are zeros);
+//   * a float per column, 1 where the column has a weight other than 0, else 0.
 constexpr uint32_t kNoSplit = 0xff7fffffu;        // -FLT_MAX, above every magnitude's bits
 constexpr uint32_t kSplitHolds = (127 - 110) << 23;  // 2^-110: larger values split without a rest
-__host__ __device__ __forceinline__ int range_tail(int c_in) { return c_in % 32 ? 0 : 4; }
-__host__ __device__ __forceinline__ uint32_t* range_word(const float* packed, int64_t layout, int c_in) {
-  return reinterpret_cast<uint32_t*>(const_cast<float*>(packed)) + layout + range_tail(c_in) - 1;
+__host__ __device__ __forceinline__ int range_tail(int c_in, int c_out) {
+  return c_in % 32 ? 0 : c_out + 4;
+}
+__host__ __device__ __forceinline__ uint32_t* range_word(const float* packed, int64_t layout, int c_in,
+                                                         int c_out) {
+  return reinterpret_cast<uint32_t*>(const_cast<float*>(packed)) + layout + range_tail(c_in, c_out) - 1;
+}
+// Padding: lane 32 + column % 32 of the column's block, the last stage's last
+// vector, one float before the range word's place in it.
+__device__ __forceinline__ float* column_flag(const float* packed, int64_t layout, int c_in, int c_out,
+                                              int column) {
+  return const_cast<float*>(packed) + layout +
+         (c_in % 32 ? -32 * c_out + column / 32 * 1024 + 3 * 256 + (32 + column % 32) * 4 + 2 : column);
 }
 
 // MFMA layout: [k][chunk][c_out/32][u][lane][16/sizeof(T)].  Lane l of a
@@ -182,25 +194,38 @@ __global__ void pack_mfma_kernel(const void* w, int w_dt, int layout, int K, int
     packed[e] = from_f32<T>(ci < c_in ? src_weight(w, w_dt, layout, K, c_in, c_out, k, ci, co)
                                       : 0.f);
   }
-  if constexpr (std::is_same<T, float>::value)  // the layout's range word (below), before its maximum
-    if (blockIdx.x == 0 && threadIdx.x == 0) *range_word(packed, total, c_in) = 0u;
+  if constexpr (std::is_same<T, float>::value)  // no column marked, no magnitude seen (padding is 0 too)
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < range_tail(c_in, c_out);
+         e += gridDim.x * blockDim.x)
+      packed[total + e] = 0.f;
 }
 
-// The range word of an f32 layer's packed weights: the bits of their largest
-// magnitude, or kNoSplit where a weight is not finite or so small that three
-// bf16 values do not hold it.  256 weights a block and step, one atomic per
-// wave.
-__global__ void __launch_bounds__(256) weight_range_kernel(const void* w, int w_dt, int64_t count,
-                                                           uint32_t* word) {
+// The range word and the column marks.  KRSC weights are [column][slot and
+// channel]: a block takes one column; flat ones end in the columns: a block takes
+// 32 of them.  One atomic per block, as they all meet in one word: packing 27 x 64
+// -> 64 takes 6.0 us with it, 24.6 with one per wave, 4.1 without the range.
+template <bool KRSC>
+__global__ void __launch_bounds__(1024) weight_range_kernel(const void* w, int w_dt, int64_t rows, int c_in,
+                                                            int c_out, float* packed, int64_t layout) {
+  constexpr int CB = KRSC ? 1 : 32, RL = 1024 / CB;
+  const int col = blockIdx.x * CB + threadIdx.x % CB;
   uint32_t most = 0;
-  for (int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x; e < count; e += (int64_t)gridDim.x * 256) {
-    const uint32_t v = __float_as_uint(load_any(w, w_dt, e)) & 0x7fffffffu;
+#pragma unroll 4
+  for (int64_t r = (int64_t)blockIdx.y * RL + threadIdx.x / CB; r < rows; r += (int64_t)gridDim.y * RL) {
+    const uint32_t v = __float_as_uint(load_any(w, w_dt, KRSC ? col * rows + r : r * c_out + col)) & 0x7fffffffu;
     const bool held = v < 0x7f800000u && (v == 0 || v >= kSplitHolds);
     most = max(most, held ? v : kNoSplit);
   }
+  if (most) *column_flag(packed, layout, c_in, c_out, col) = 1.f;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) most = max(most, static_cast<uint32_t>(__shfl_xor(most, off, kWave)));
-  if ((threadIdx.x & 63) == 0) atomicMax(word, most);
+  __shared__ uint32_t s_most[1024 / kWave];
+  if (threadIdx.x % kWave == 0) s_most[threadIdx.x / kWave] = most;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (const uint32_t m : s_most) most = max(most, m);
+    atomicMax(range_word(packed, layout, c_in, c_out), most);
+  }
 }
 
 // The direct-to-LDS kernel's output rows are written once and not read
@@ -330,8 +355,8 @@ template <> struct MfmaOp<float> {
 //     For features that is at most max|w| 2^-134 for each of up to 2^18
 //     products, so sums of at least max|w| 2^-88 have it below 2^-28 of them,
 //     and smaller ones are computed again (max|w| from the range word of the
-//     packed weights).  A sum of exactly zero is, where its row gathers a value
-//     so small that all three parts may vanish.
+//     packed weights).  A sum of exactly zero is, where its column has weights
+//     and its row gathers a value so small that all three parts may vanish.
 //   * Layers with such weights run on the f32 unit throughout: nothing bounds
 //     the features that would multiply their errors.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -404,27 +429,46 @@ __device__ __forceinline__ float split_limit(uint32_t range) {
 
 // Bit r set: row r of a 32-row block is in `rows` and gathers a value other than
 // zero below 2^-132, which the split may turn into nothing.  s_orow: the block's
-// output rows; first: its first processing position.
+// output rows; first: its first processing position.  Sixteen lanes read a row,
+// four rows of a wave and four slots at a time.
 __device__ uint32_t vanishing_rows(const float* __restrict__ feat, int c_in,
                                    const int32_t* __restrict__ nbr, int nbr_ordered, int64_t n_out,
                                    int K, const int32_t* s_orow, int64_t first, uint32_t rows) {
   constexpr uint32_t kVanishing = (1u << 17) << 1;  // 2^-132's bits, shifted left
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
-  const int32_t o = s_orow[r];
-  bool any = false;
-  if (o >= 0 && ((rows >> r) & 1)) {
-    for (int k = 0; k < K; ++k) {
-      const int32_t j = nbr ? nbr[(int64_t)k * n_out + (nbr_ordered ? first + r : (int64_t)o)] : o;
-      if (j < 0) continue;
-      const uint4* src = reinterpret_cast<const uint4*>(feat + (int64_t)j * c_in);
-      for (int c = h; c < c_in / 4; c += 2) {
-        const uint4 v = src[c];
-        for (const uint32_t x : {v.x, v.y, v.z, v.w}) any |= (x << 1) - 1u < kVanishing - 1u;
+  constexpr int G = 4;
+  const int lane = threadIdx.x & 63, group = lane >> 4, piece = lane & 15;
+  uint32_t found = 0;
+  for (int i = 0; i < 32; i += 4) {
+    if (((rows >> i) & 15u) == 0) continue;
+    const int r = i + group;
+    const int32_t o = s_orow[r];
+    const bool look = o >= 0 && ((rows >> r) & 1);
+    bool any = false;
+    for (int k0 = 0; k0 < K; k0 += G) {
+      int32_t j[G];
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        j[u] = -1;
+        if (look && k0 + u < K)
+          j[u] = nbr ? nbr[(int64_t)(k0 + u) * n_out + (nbr_ordered ? first + r : (int64_t)o)] : o;
+      }
+      for (int c = piece; c < c_in / 4; c += 16) {
+        uint4 v[G];
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+          v[u] = j[u] >= 0 ? reinterpret_cast<const uint4*>(feat + (int64_t)j[u] * c_in)[c]
+                           : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+          any |= (v[u].x << 1) - 1u < kVanishing - 1u || (v[u].y << 1) - 1u < kVanishing - 1u ||
+                 (v[u].z << 1) - 1u < kVanishing - 1u || (v[u].w << 1) - 1u < kVanishing - 1u;
       }
     }
+    const uint64_t b = __ballot(any);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) found |= ((b >> (16 * g)) & 0xffffu) ? 1u << (i + g) : 0u;
   }
-  const uint64_t b = __ballot(any);
-  return static_cast<uint32_t>(b) | static_cast<uint32_t>(b >> 32);
+  return found;
 }
 
 // The elements of this lane's accumulators that the f32 unit computes again (see
@@ -460,14 +504,19 @@ struct Redo {
         for (int i = 0; i < 16; ++i)
           if (rb * 32 + (i >> 2) * 8 + h * 4 + (i & 3) >= left) acc[rb][nb][i] = 1.f;
   }
-  // rows of block rb with an element of exactly zero, as row bits
-  static __device__ __forceinline__ uint32_t zero_rows(const f32x16 (&acc)[NB]) {
+  // rows of one block with an element of exactly zero in a column that has
+  // weights, as row bits.  flag: this lane's column of the first block's mark.
+  static __device__ __forceinline__ uint32_t zero_rows(const f32x16 (&acc)[NB], const float* flag,
+                                                       int flag_stride) {
+    bool live[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) live[nb] = flag[nb * flag_stride] != 0.f;
     uint32_t rows = 0;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       bool zero = false;
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) zero |= acc[nb][i] == 0.f;
+      for (int nb = 0; nb < NB; ++nb) zero |= acc[nb][i] == 0.f && live[nb];
       const uint64_t b = __ballot(zero);
       const int r = (i >> 2) * 8 + (i & 3);
       rows |= (static_cast<uint32_t>(b) ? 1u << r : 0u) | (static_cast<uint32_t>(b >> 32) ? 16u << r : 0u);
@@ -575,7 +624,7 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
   const int nbt = static_cast<int>(item % ncol);
   const int nch = (c_in + CK - 1) / CK;  // C_in % 16 == 0: the last chunk may be half padding
   uint32_t range = 0;  // f32: asked for here, used after the set-up
-  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in);
+  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in, c_out);
 
   // ---- tile set-up: output rows, their slot lists and slot masks.  The map
   // entries are read 32 slots at a time, all in flight before any is used
@@ -893,10 +942,12 @@ __global__ void __launch_bounds__(256, 2) conv_mfma_kernel(
       if (no_split) {
         bad.all();
       } else {
+        const float* const flag = column_flag(W, (int64_t)K * nch * CK * c_out, c_in, c_out, nbt * BN + (lane & 31));
+        const int flag_stride = c_in % 32 ? 1024 : 32;
         uint32_t vanish[2];
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb) {
-          const uint32_t zeros = Redo<2, NB>::zero_rows(acc[rb]);
+          const uint32_t zeros = Redo<2, NB>::zero_rows(acc[rb], flag, flag_stride);
           vanish[rb] = zeros ? vanishing_rows(feat, c_in, nbr, nbr_ordered, n_out, K,
                                               s_orow + wave * 64 + rb * 32, tile0 + wave * 64 + rb * 32,
                                               zeros)
@@ -1022,7 +1073,7 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
   const int nbt = static_cast<int>(item % ncol);
   const int nch = c_in / CK;
   uint32_t range = 0;
-  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in);
+  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in, c_out);
 
   // ---- tile set-up: output rows and slot masks (the entries themselves are
   // loaded again stage by stage), as in conv_mfma_kernel; thread t < TR
@@ -1436,10 +1487,12 @@ __global__ void __launch_bounds__(256, 2) conv_dma_kernel(
       if (no_split) {
         bad.all();
       } else {
+        const float* const flag = column_flag(W, (int64_t)K * nch * CK * c_out, c_in, c_out, nbt * BN + (lane & 31));
+        const int flag_stride = c_in % 32 ? 1024 : 32;
         uint32_t vanish[RB];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-          const uint32_t zeros = Redo<RB, NB>::zero_rows(acc[rb]);
+          const uint32_t zeros = Redo<RB, NB>::zero_rows(acc[rb], flag, flag_stride);
           vanish[rb] = zeros ? vanishing_rows(feat, c_in, nbr, nbr_ordered, n_out, K,
                                               s_orow + wave * WR + rb * 32, tile0 + wave * WR + rb * 32,
                                               zeros)
@@ -1517,7 +1570,7 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
   const int nbt = static_cast<int>(item % ncol);
   const int nch = (c_in + CK - 1) / CK;
   uint32_t range = 0;
-  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in);
+  if constexpr (F32) range = *range_word(W, (int64_t)K * nch * CK * c_out, c_in, c_out);
 
   // ---- set-up: wave w reads the map entries of its own slots for the 64
   // rows, sixteen slots at a time, all in flight before any is used; a map
@@ -1775,10 +1828,12 @@ __global__ void __launch_bounds__(256, 2) conv_split_kernel(
     if (no_split) {
       bad.all();
     } else if (wave == 0) {
+      const float* const flag = column_flag(W, (int64_t)K * nch * CK * c_out, c_in, c_out, nbt * BN + (lane & 31));
+      const int flag_stride = c_in % 32 ? 1024 : 32;
       uint32_t vanish[2];
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
-        const uint32_t zeros = Redo<2, NB>::zero_rows(acc[rb]);
+        const uint32_t zeros = Redo<2, NB>::zero_rows(acc[rb], flag, flag_stride);
         vanish[rb] = zeros ? vanishing_rows(feat, c_in, nbr, nbr_ordered, n_out, K, s_orow + rb * 32,
                                             tile0 + rb * 32, zeros)
                            : 0u;
@@ -2437,7 +2492,7 @@ extern "C" int64_t tsc_packed_weight_bytes(int32_t k_vol, int32_t c_in, int32_t 
   if (pick_path(dtype, c_in, c_out, k_vol) == kMfma) {
     const int ck = pick_ck(dtype, c_in);
     return ((int64_t)k_vol * mfma_chunks(c_in, ck) * ck * c_out +
-            (dtype == TSC_F32 ? range_tail(c_in) : 0)) * dtype_bytes(dtype);
+            (dtype == TSC_F32 ? range_tail(c_in, c_out) : 0)) * dtype_bytes(dtype);
   }
   const int64_t bytes = narrow_bytes(dtype, k_vol, c_in, c_out);
   // widths that do not fill their pieces and tiles: no less than an fp32
@@ -2481,9 +2536,14 @@ extern "C" int tsc_pack_weight(const void* w, int32_t w_dtype, int32_t layout, i
     if (dtype == TSC_F32) {
       float* const p = static_cast<float*>(packed);
       pack_mfma_kernel<float><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out, ck, p);
-      const int64_t count = (int64_t)k_vol * c_in * c_out;
-      weight_range_kernel<<<static_cast<unsigned>(std::min<int64_t>(ceil_div(count, 1024), 1024)), 256, 0, s>>>(
-          w, w_dtype, count, range_word(p, (int64_t)k_vol * mfma_chunks(c_in, ck) * ck * c_out, c_in));
+      const int64_t rows = (int64_t)k_vol * c_in;
+      const int64_t elems = (int64_t)k_vol * mfma_chunks(c_in, ck) * ck * c_out;
+      if (layout == 0)
+        weight_range_kernel<true><<<dim3(c_out, static_cast<unsigned>(std::min<int64_t>(ceil_div(rows, 8192), 16))),
+                                    1024, 0, s>>>(w, w_dtype, rows, c_in, c_out, p, elems);
+      else
+        weight_range_kernel<false><<<dim3(c_out / 32, static_cast<unsigned>(std::min<int64_t>(ceil_div(rows, 256), 64))),
+                                     1024, 0, s>>>(w, w_dtype, rows, c_in, c_out, p, elems);
     } else if (dtype == TSC_F16)
       pack_mfma_kernel<__half><<<grid, 256, 0, s>>>(w, w_dtype, layout, k_vol, c_in, c_out, ck,
                                                     static_cast<__half*>(packed));
